@@ -1,6 +1,7 @@
 /*
  * mfa.h -- C ABI of the MI355X (gfx950) flash-attention library
- * (libmtlfa_hip.so, built from mtlflashattn_amd/csrc/mfa_fwd.hip and mfa_bwd.hip).
+ * (libmtlfa_hip.so, built from mtlflashattn_amd/csrc/mfa_fwd.hip, mfa_bwd.hip and
+ * mfa_merge.hip).
  *
  * This is the drop-in boundary that replaces the reference's per-tier Metal
  * launch calls.  In the reference the Python launcher binds a JIT-compiled
@@ -310,6 +311,37 @@ int64_t mfa_bwd_workspace_bytes(const mfa_bwd_params* params);
  * caller.  Never synchronizes, never allocates. */
 int mfa_bwd(const mfa_bwd_params* params, void* workspace, int64_t workspace_bytes, void* stream);
 int mfa_bwd_params_size(void);
+
+/*
+ * Merge of attention partials of the same queries over disjoint key sets
+ * (context-parallel shards, cache + new tokens).  No counterpart in the
+ * reference.  Part i holds o [batch, seqlen, heads, head_dim] (16-byte
+ * aligned, head dim contiguous, element strides in multiples of 16 bytes) and
+ * its log-sum-exp lse [batch, heads, seqlen] (fp32, any element strides).
+ *   lse_out = ln(sum_i exp(lse_i)), out = sum_i exp(lse_i - lse_out) o_i,
+ * both contiguous ([batch, seqlen, heads, head_dim] in `dtype`, the parts'
+ * element type, and [batch, heads, seqlen] fp32); a row whose merged lse is
+ * infinite (no key in any part) gets weights of 0.  Sums in fp32, in part
+ * order.  head_dim is a multiple of 16 bytes.  Enqueues one kernel on
+ * `stream`; never synchronizes, never allocates.
+ */
+#define MFA_MERGE_MAX_PARTS 16
+typedef struct mfa_merge_part {
+    const void* o;
+    const float* lse;
+    int64_t o_batch_stride, o_seq_stride, o_head_stride;
+    int64_t lse_batch_stride, lse_head_stride, lse_seq_stride;
+} mfa_merge_part;
+typedef struct mfa_merge_params {
+    mfa_merge_part part[MFA_MERGE_MAX_PARTS];
+    void* out;
+    float* lse_out;
+    int32_t parts;
+    int32_t dtype; /* MFA_DTYPE_* */
+    int32_t batch, seqlen, heads, head_dim;
+} mfa_merge_params;
+int mfa_merge(const mfa_merge_params* params, void* stream);
+int mfa_merge_params_size(void);
 
 #ifdef __cplusplus
 }

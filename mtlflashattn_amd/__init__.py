@@ -294,10 +294,15 @@ def merge_attention_partials(outs, lses):
     w_i = exp(lse_i - lse), lse = ln(sum_i exp(lse_i)); rows without a valid
     key in any part get out = 0, lse = -inf.  This is the merge a
     context-parallel forward (key/value shards on different GPUs) or a
-    cache + new-token split needs; it runs as PyTorch elementwise ops.
+    cache + new-token split needs.  On a ROCm GPU it is one HIP launch
+    (mfa_merge); where gradients are recorded, and for inputs that kernel does
+    not take, it runs as PyTorch elementwise ops.
     """
     if len(outs) != len(lses) or not outs:
         raise ValueError("mtlflashattn_amd: merge_attention_partials needs matching, non-empty outs and lses")
+    merged = _kernel.merge_partials(outs, lses)
+    if merged is not None:
+        return merged
     lse_all = torch.stack([x.float() for x in lses])
     lse = torch.logsumexp(lse_all, dim=0)
     safe = torch.where(torch.isinf(lse), torch.zeros_like(lse), lse)

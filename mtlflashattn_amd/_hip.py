@@ -80,6 +80,29 @@ class MfaBwdParams(ctypes.Structure):
     ]
 
 
+MFA_MERGE_MAX_PARTS = 16
+
+
+class MfaMergePart(ctypes.Structure):
+    """Mirror of `mfa_merge_part` (include/mfa.h)."""
+
+    _fields_ = [
+        ("o", _c_ptr), ("lse", _c_ptr),
+        ("o_batch_stride", _c_i64), ("o_seq_stride", _c_i64), ("o_head_stride", _c_i64),
+        ("lse_batch_stride", _c_i64), ("lse_head_stride", _c_i64), ("lse_seq_stride", _c_i64),
+    ]
+
+
+class MfaMergeParams(ctypes.Structure):
+    """Mirror of `mfa_merge_params` (include/mfa.h)."""
+
+    _fields_ = [
+        ("part", MfaMergePart * MFA_MERGE_MAX_PARTS), ("out", _c_ptr), ("lse_out", _c_ptr),
+        ("parts", _c_i32), ("dtype", _c_i32),
+        ("batch", _c_i32), ("seqlen", _c_i32), ("heads", _c_i32), ("head_dim", _c_i32),
+    ]
+
+
 class MfaLaunchInfo(ctypes.Structure):
     """Mirror of `mfa_launch_info` (include/mfa.h)."""
 
@@ -148,6 +171,10 @@ def load():
         lib.mfa_bwd_workspace_bytes.argtypes = [ctypes.POINTER(MfaBwdParams)]
         lib.mfa_bwd.restype = ctypes.c_int
         lib.mfa_bwd.argtypes = [ctypes.POINTER(MfaBwdParams), _c_ptr, ctypes.c_int64, _c_ptr]
+        lib.mfa_merge_params_size.restype = ctypes.c_int
+        lib.mfa_merge_params_size.argtypes = []
+        lib.mfa_merge.restype = ctypes.c_int
+        lib.mfa_merge.argtypes = [ctypes.POINTER(MfaMergeParams), _c_ptr]
         if lib.mfa_abi_version() != MFA_ABI_VERSION:
             raise HipLibraryError(
                 f"mtlflashattn_amd: {path} has ABI {lib.mfa_abi_version()}, expected {MFA_ABI_VERSION}; rebuild it"
@@ -156,6 +183,11 @@ def load():
             raise HipLibraryError(
                 f"mtlflashattn_amd: mfa_bwd_params is {lib.mfa_bwd_params_size()} bytes in {path} but "
                 f"{ctypes.sizeof(MfaBwdParams)} in the ctypes mirror; rebuild it"
+            )
+        if lib.mfa_merge_params_size() != ctypes.sizeof(MfaMergeParams):
+            raise HipLibraryError(
+                f"mtlflashattn_amd: mfa_merge_params is {lib.mfa_merge_params_size()} bytes in {path} but "
+                f"{ctypes.sizeof(MfaMergeParams)} in the ctypes mirror; rebuild it"
             )
         if lib.mfa_params_size() != ctypes.sizeof(MfaFwdParams):
             raise HipLibraryError(
@@ -229,6 +261,13 @@ def bwd(params: MfaBwdParams, workspace: int, workspace_bytes_: int, stream: int
     rc = lib.mfa_bwd(ctypes.byref(params), _c_ptr(workspace), int(workspace_bytes_), _c_ptr(stream))
     if rc != MFA_OK:
         raise HipLibraryError(lib.mfa_last_error().decode(errors="replace") or f"mfa_bwd failed ({rc})")
+
+
+def merge(params: MfaMergeParams, stream: int) -> None:
+    lib = load()
+    rc = lib.mfa_merge(ctypes.byref(params), _c_ptr(stream))
+    if rc != MFA_OK:
+        raise HipLibraryError(lib.mfa_last_error().decode(errors="replace") or f"mfa_merge failed ({rc})")
 
 
 def launch_info(params: MfaFwdParams) -> MfaLaunchInfo:

@@ -637,6 +637,70 @@ class _FlashAttnVarlenFn(torch.autograd.Function):
         return dq[0], dk[0], dv[0], None, None, None, None, None, None, None, None, None, None, None
 
 
+def _plain(*tensors) -> bool:
+    """No transform or mode sees these tensors' operations: ordinary tensors
+    (no subclass), outside vmap and the other functorch transforms,
+    forward-mode AD, dispatch / function modes and graph capture by a tracer.
+    Only then may a kernel launch stand in for a sequence of torch ops."""
+    return (
+        all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+        and torch._C._functorch.peek_interpreter_stack() is None
+        and torch.autograd.forward_ad._current_level < 0
+        and torch._C._len_torch_dispatch_stack() == 0
+        and not torch._C._is_torch_function_mode_enabled()
+        and not torch.jit.is_tracing()
+        and not torch.compiler.is_compiling()
+    )
+
+
+def merge_partials(outs, lses):
+    """(out, lse) of the merge of attention partials in one HIP launch, or
+    None where the caller's torch ops have to run: gradients are recorded, a
+    transform is active, tensors not on one ROCm GPU, layouts, types or counts
+    that mfa_merge does not take.  outs: [(B,) L, H, D], lses: [(B,) H, L]."""
+    n = len(outs)
+    o0 = outs[0]
+    if not 1 <= n <= _hip.MFA_MERGE_MAX_PARTS or not all(torch.is_tensor(t) for t in (*outs, *lses)):
+        return None
+    if not _plain(*outs, *lses) or _needs_grad(*outs, *lses):
+        return None
+    dim, dt, dev = o0.dim(), o0.dtype, o0.device
+    if dim not in (3, 4) or dt not in _SUPPORTED_DTYPES or not _is_rocm_tensor(o0) or o0.numel() == 0:
+        return None
+    lshape = (*o0.shape[:-3], o0.shape[-2], o0.shape[-3])
+    if o0.shape[-1] % (4 if dt == torch.float32 else 8) or not o0.is_contiguous():
+        return None
+    for o, l in zip(outs, lses):
+        if (o.shape != o0.shape or o.dtype != dt or o.device != dev or not _fits_abi(o)
+                or l.shape != lshape or l.dtype != torch.float32 or l.device != dev):
+            return None
+    out = torch.empty(o0.shape, dtype=dt, device=dev)
+    lse = torch.empty(lshape, dtype=torch.float32, device=dev)
+    p = _hip.MfaMergeParams()
+    for part, o, l in zip(p.part, outs, lses):
+        part.o, part.lse = o.data_ptr(), l.data_ptr()
+        if dim == 4:
+            part.o_batch_stride, part.o_seq_stride, part.o_head_stride, _ = o.stride()
+            part.lse_batch_stride, part.lse_head_stride, part.lse_seq_stride = l.stride()
+        else:
+            part.o_seq_stride, part.o_head_stride, _ = o.stride()
+            part.lse_head_stride, part.lse_seq_stride = l.stride()
+        # (a size-1 dim may carry any stride)
+        if o.shape[-3] == 1:
+            part.o_seq_stride = 0
+        if o.shape[-2] == 1:
+            part.o_head_stride = 0
+        if dim == 4 and o.shape[0] == 1:
+            part.o_batch_stride = 0
+    p.out, p.lse_out = out.data_ptr(), lse.data_ptr()
+    p.parts, p.dtype = n, _hip.DTYPE_CODES[dt]
+    p.batch = o0.shape[0] if dim == 4 else 1
+    p.seqlen, p.heads, p.head_dim = o0.shape[-3:]
+    with torch.cuda.device(dev):
+        _hip.merge(p, torch._C._cuda_getCurrentRawStream(dev.index))
+    return out, lse
+
+
 def split_chunk(q, k):
     """Split-KV chunk (keys) the library picks for heads-third q/k (0: single pass)."""
     if q.dtype == torch.float32:
