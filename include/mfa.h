@@ -271,9 +271,9 @@ int mfa_fwd_splitkv_static(const mfa_fwd_params* params, int32_t split_keys, voi
  * Deterministic (no atomics): one kernel owns each dK/dV block and loops over
  * every query of its K/V head; another owns each dQ block.
  * fp32 (dtype_in = MFA_DTYPE_F32: q, k, v, o, dout and the gradients fp32)
- * runs fp32 kernels on the vector ALU with the fp32 forward's score transform
- * (strides then multiples of 4 elements; the workspace holds the row sums
- * only).  bf16/fp16 run on the matrix cores.
+ * runs fp32 kernels on the fp32 matrix cores with the fp32 forward's score
+ * transform (strides then multiples of 4 elements; the workspace holds the row
+ * sums only).
  */
 typedef struct mfa_bwd_params {
     /* q, k, v, o (the forward output), shapes, strides, masks and biases as

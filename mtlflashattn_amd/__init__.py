@@ -8,7 +8,7 @@ approximating (metal_flash_attn/__init__.py:1-5).
 Backward: the reference is inference-only (metal_flash_attn/__init__.py:3-4).
 Here calls whose inputs require grad are differentiable through HIP
 backward kernels (dq, dk, dv; the returned lse too): bf16/fp16 on the matrix
-cores, fp32 in fp32 on the vector ALU.  Paged K/V stay forward-only: their
+cores, fp32 in fp32 on the fp32 matrix cores.  Paged K/V stay forward-only: their
 backward raises NotImplementedError, as do dropout_p > 0, deterministic=True
 and return_attn_probs=True.
 

@@ -16,6 +16,8 @@
 // Thread-local message buffer behind mfa_last_error() (512 bytes, defined in
 // mfa_fwd.hip), shared by every entry point of the library.
 __attribute__((visibility("hidden"))) char* mfa_error_buffer();
+// Compute units of the device `stream` (a hipStream_t) belongs to (mfa_fwd.hip).
+__attribute__((visibility("hidden"))) int mfa_chip_cus(void* stream);
 
 namespace {
 

@@ -2920,6 +2920,7 @@ int static_scratch(hipStream_t st, void** out) {
 }  // namespace
 
 char* mfa_error_buffer() { return g_err; }
+int mfa_chip_cus(void* stream) { return chip_geometry_of(static_cast<hipStream_t>(stream)).cus; }
 
 extern "C" {
 
