@@ -1,7 +1,6 @@
 /*
  * mfa.h -- C ABI of the MI355X (gfx950) flash-attention library
- * (libmtlfa_hip.so, built from mtlflashattn_amd/csrc/mfa_fwd.hip, mfa_bwd.hip and
- * mfa_merge.hip).
+ * (libmtlfa_hip.so, built from the sources in mtlflashattn_amd/csrc).
  *
  * This is the drop-in boundary that replaces the reference's per-tier Metal
  * launch calls.  In the reference the Python launcher binds a JIT-compiled
@@ -55,9 +54,9 @@ extern "C" {
 #define MFA_MAX_HEAD_DIM 128
 
 /* tile_hint values (bf16/fp16 only; fp32 has one kernel).  Sequences of one
- * query row (and single-row grouped-query decode, whose query heads are
- * computed as the rows of one K/V head) always run the exact-row kernel,
- * whose probabilities carry two 16-bit terms; the hint applies to the rest. */
+ * query row always run the single-row kernel, which computes the query heads
+ * of a K/V head together and whose probabilities carry two 16-bit terms; the
+ * hint applies to the rest. */
 #define MFA_TILE_AUTO 0     /* library's choice */
 #define MFA_TILE_256 1      /* 256-row tiles, 4 wavefronts */
 #define MFA_TILE_PINGPONG 2 /* ping-pong tiles, 8 wavefronts: 512 rows at head_dim <= 64,
@@ -166,7 +165,7 @@ typedef struct mfa_fwd_params {
 
     /* Varlen calls, optional (0 = unknown; ABI 7): 1 when the caller knows
      * that no sequence has exactly one query row.  A varlen call otherwise
-     * adds a launch of the exact-row kernel for such sequences (the main
+     * adds a launch of the single-row kernel for such sequences (the main
      * launch leaves them to it); 1 skips that launch, so a sequence of one
      * query row would keep its o rows (and lse) unwritten.  Ignored by dense
      * calls.  No counterpart in the reference. */
@@ -232,7 +231,11 @@ int mfa_params_size(void);
  * 256-byte aligned device buffer of at least that many bytes, owned by the
  * caller and reused only after the call's kernels ran (stream order).
  * split_keys must be 0 (same as mfa_fwd) or a positive multiple of 64 (of
- * 256 with a block_table).  softmax_lse and block_table work as in mfa_fwd. */
+ * 256 with a block_table).  Sequences of one query row are chunked by the
+ * library, from their own key count, in every entry point alike: there
+ * split_keys != 0 only offers the workspace (0 bytes where a workgroup per
+ * sequence and K/V head walking all chunks is faster), and the results of
+ * mfa_fwd and mfa_fwd_splitkv are the same bits.  softmax_lse and block_table work as in mfa_fwd. */
 int32_t mfa_fwd_split_keys(const mfa_fwd_params* params);
 int64_t mfa_fwd_workspace_bytes(const mfa_fwd_params* params, int32_t split_keys);
 int mfa_fwd_splitkv(const mfa_fwd_params* params, int32_t split_keys, void* workspace, int64_t workspace_bytes,

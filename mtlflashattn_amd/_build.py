@@ -21,6 +21,7 @@ REPO_DIR = os.path.dirname(PKG_DIR)
 # picks, which otherwise moves them between register files every block)
 SRCS = [
     (os.path.join(PKG_DIR, "csrc", "mfa_fwd.hip"), []),
+    (os.path.join(PKG_DIR, "csrc", "mfa_decode.hip"), ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]),
     (os.path.join(PKG_DIR, "csrc", "mfa_bwd.hip"), ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]),
     (os.path.join(PKG_DIR, "csrc", "mfa_bwd32.hip"), ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]),
     (os.path.join(PKG_DIR, "csrc", "mfa_merge.hip"), []),

@@ -218,7 +218,7 @@ def _run(q, k, v, out, *, scale, causal, softcap, window_left, window_right, ali
     are then [num_pages, page_block_size, Hkv, D] and every sequence's key
     count comes from seqlen_k (dense) or cu_k (varlen).
     no_single_rows: (varlen) no sequence has exactly one query row, so the
-    exact-row launch for such sequences is skipped.
+    single-row launch for such sequences is skipped.
     """
     _kernel_mode()
     B, Sq, Hq, D = q.shape
@@ -325,6 +325,7 @@ def _prepare(q, k, v, out, batch, Hq, Hkv, Lq, Lk, Dp, varlen, scale, causal, so
              has_alibi, alibi_bstride, lse_strides=None, paged=None):
     """(parameter template without data pointers, split-KV choice) of a call."""
     p = _hip.MfaFwdParams()
+    p.q = p.k = p.v = p.o = 256  # placeholders: the choice below reads no tensor
     p.q_batch_stride, p.q_seq_stride, p.q_head_stride = _strides_bsh(q)
     p.k_batch_stride, p.k_seq_stride, p.k_head_stride = _strides_bsh(k)
     p.v_batch_stride, p.v_seq_stride, p.v_head_stride = _strides_bsh(v)
@@ -350,14 +351,26 @@ def _prepare(q, k, v, out, batch, Hq, Hkv, Lq, Lk, Dp, varlen, scale, causal, so
     if paged is not None:
         p.block_table_batch_stride, p.page_block_size, p.num_pages = paged
     chunk = _split_choice(p, q.dtype, hint)
-    p.cu_seqlens_q = p.cu_seqlens_k = p.alibi_slopes = None
+    p.q = p.k = p.v = p.o = p.cu_seqlens_q = p.cu_seqlens_k = p.alibi_slopes = None
     return p, chunk
 
 
 def _split_choice(p, dtype, hint):
     if dtype == torch.float32 or hint in _PP_HINTS:
         return 0
-    return _hip.split_keys(p) if _SPLIT_KEYS is None else _SPLIT_KEYS
+    if _SPLIT_KEYS is not None:
+        return _SPLIT_KEYS
+    chunk = _hip.split_keys(p)
+    if p.seqlen_q == 1 and (chunk or p.seqlen_k <= _SINGLE_ROW_SPLIT * _MAX_SPLITS):
+        # single rows: the library chunks each sequence by its own length,
+        # and says through the workspace whether it splits this call
+        return _SINGLE_ROW_SPLIT if _hip.workspace_bytes(p, _SINGLE_ROW_SPLIT) else 0
+    return chunk
+
+
+# the chunk of a split request for single-row calls (any valid one: theirs is
+# the library's) and the most chunks such a request may imply
+_SINGLE_ROW_SPLIT, _MAX_SPLITS = 2048, 1024
 
 
 def _launch(p, chunk, device):
@@ -463,7 +476,7 @@ def forward_varlen(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap=0.0
     (paged calls are forward-only).  Inputs that require grad (and no block
     table, q.dtype output) go through the HIP backward.  no_single_rows: the
     caller knows no sequence has exactly one query row (the library then
-    skips the exact-row launch for such sequences; a one-row sequence would
+    skips the single-row launch for such sequences; a one-row sequence would
     be left unwritten).
     """
     batch = cu_q.shape[0] - 1

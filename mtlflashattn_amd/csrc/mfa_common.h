@@ -53,16 +53,9 @@ struct KArgs {
     float softcap_k;  // 2 * log2(e) / softcap
     float softcap_sk; // scale * softcap_k (the soft-cap of a raw score in one exponent)
     int32_t wl, wr, causal;
-    int32_t decode_pack;  // rows are the query heads of one K/V head (single-row GQA decode)
-    // varlen: element strides between the tokens of q / o at which sequences
-    // start, and query rows per token (pack_r = query heads per K/V head when
-    // packed, else 1; rows then step by qs / os)
-    int64_t qts, ots;
-    int32_t pack_r;
-    // sequences of one query row (varlen calls that mix them with longer
-    // ones): 0 = every sequence is this launch's, 1 = this launch skips them
-    // (the exact-row kernel's launch computes them), 2 = this launch (the
-    // exact-row kernel) computes only them
+    // varlen calls that may mix sequences of one query row with longer ones:
+    // 1 = this launch skips the former (the single-row kernel's launch
+    // computes them)
     int32_t single_rows;
     // ping-pong tiles packing the query heads of one K/V head (grouped-query
     // calls): hpack heads share a tile and its K/V stream, each taking
@@ -145,14 +138,22 @@ __device__ __forceinline__ float sum_halves(float x) {
 // holds afterwards (the asm only reads it), so M0 is neither written by the
 // asm nor in its clobber list.  (s_nop 0: one wait state between the M0
 // write and the load that reads it.)
+// NT: a non-temporal load, for data that no other workgroup reads.
+template <bool NT = false>
 __device__ __forceinline__ void lds_load16(uint64_t base, uint32_t bytes, uint16_t* dst, uint32_t off) {
     typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t rsrc_t;
     const rsrc_t r = {(uint32_t)base, (uint32_t)(base >> 32) & 0xffffu, bytes, (uint32_t)kBufferDword3};
     const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)dst;
-    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
-                 :
-                 : "v"(off), "s"(r), "{m0}"(lds)
-                 : "memory");
+    if constexpr (NT)
+        asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen nt lds"
+                     :
+                     : "v"(off), "s"(r), "{m0}"(lds)
+                     : "memory");
+    else
+        asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+                     :
+                     : "v"(off), "s"(r), "{m0}"(lds)
+                     : "memory");
 }
 
 // Compile-time loop: f(std::integral_constant<int, I>{}) for I = 0 .. N-1.
@@ -265,14 +266,14 @@ __device__ __forceinline__ SeqView seq_view(const KArgs& a, int b, int hq) {
     if (a.cu_q) {
         const int q_start = a.cu_q[b];
         const int k_start = a.cu_k[b];
-        s.Lq = (a.cu_q[b + 1] - q_start) * a.pack_r;
+        s.Lq = a.cu_q[b + 1] - q_start;
         s.Lk = a.cu_k[b + 1] - k_start;
-        qo = (int64_t)q_start * a.qts;
+        qo = (int64_t)q_start * a.qs;
         ko = a.bt ? 0 : (int64_t)k_start;  // paged: pages come from the table
         s.q = a.q + (qo + (int64_t)hq * a.qh) * ES;
         s.k = a.k + (ko * a.ks + (int64_t)hkv * a.kh) * ES;
         s.v = a.v + (ko * a.vs + (int64_t)hkv * a.vh) * ES;
-        s.o = a.o + ((int64_t)q_start * a.ots + (int64_t)hq * a.oh) * OES;
+        s.o = a.o + ((int64_t)q_start * a.os + (int64_t)hq * a.oh) * OES;
         s.lse = a.lse ? a.lse + (int64_t)hq * a.lse_h + q_start : nullptr;
     } else {
         s.Lq = a.Lq;

@@ -5,12 +5,11 @@
 // states the mask/bias/online-softmax math most plainly) and :1165-1208 (the
 // chunked fp32 torch path, whose results these kernels must reproduce).
 //
-// Kernels: mfa_fwd16_kernel (bf16/fp16, 4 wavefronts; its EXACT
-// instantiation serves single query rows with two-term probabilities),
-// mfa_fwd16_pp_kernel (bf16/fp16, 8 wavefronts on a ping-pong schedule: the
-// two wavefronts of a SIMD alternate MFMA and softmax phases),
-// mfa_fwd16_tk_kernel (at most 32 keys per sequence), mfa_fwd32_kernel
-// (fp32) and mfa_combine_kernel (split-KV merge).  Grouped-query calls pack
+// Kernels: mfa_fwd16_kernel (bf16/fp16, 4 wavefronts), mfa_fwd16_pp_kernel
+// (bf16/fp16, 8 wavefronts on a ping-pong schedule: the two wavefronts of a
+// SIMD alternate MFMA and softmax phases), mfa_fwd16_tk_kernel (at most 32 keys
+// per sequence), mfa_fwd32_kernel (fp32) and mfa_combine_kernel (split-KV
+// merge); single query rows (bf16/fp16) run mfa_decode.hip's.  Grouped-query calls pack
 // the query heads of one K/V head into a tile (each wavefront still holds
 // 32 aligned positions of one head).  Shared design:
 //  * The score tile is computed TRANSPOSED, S^T = K * Q^T, with
@@ -62,6 +61,7 @@
 
 #include "mfa.h"
 #include "mfa_common.h"
+#include "mfa_decode.h"
 
 namespace {
 
@@ -265,9 +265,7 @@ __device__ __forceinline__ float qb_max(const f32x16_t (&s)[NKB]) {
 // final O/l is unaffected.  The exponent offset mu = m*c and thr change only
 // on a move, so a block that moves no row costs one compare per row.  Rows
 // with no valid key so far keep m = thr = -inf and mu = 0, so masked scores
-// give p = 0.  With tau = 0 a row whose max did not grow gets
-// alpha = exp2(0) = 1 exactly, so each row's arithmetic is independent of
-// the other rows of its wave.
+// give p = 0.
 __device__ __forceinline__ void row_reset(RowState& rs) {
     rs.m = -INFINITY;
     rs.thr = -INFINITY;
@@ -395,44 +393,6 @@ __device__ __forceinline__ float qb_sum16(const u32x4_t (&pw)[NKB][2]) {
                 }
             }
     return acc[0] + acc[1];
-}
-
-// Two-term 16-bit probabilities, for rows whose O averages so many
-// near-equal weights that one 16-bit rounding of each weight is visible
-// against max|O| (single-row sequences and packed grouped-query decode rows):
-// hi = round16(p) and lo = round16(p - hi) (the difference is exact in fp32).
-// The PV MFMA consumes both against the same V fragment, so the weights carry
-// about 16 mantissa bits instead of 8 (bf16) or 11 (fp16).  The row sum adds
-// the fp32 weights themselves (two chains, acc[0] and acc[1]), which hi + lo
-// reproduce to 2^-17 relative (plain adds: two dot2 per pair measured 1.2%
-// slower on single-row decode).
-// One group: the 8 weights of accumulator registers 8*st..8*st+7.
-template <bool IS_BF16>
-__device__ __forceinline__ void probs16x2_group(const f32x16_t& s, int st, u32x4_t& ph, u32x4_t& pl,
-                                                float (&acc)[2], float mu, float c) {
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        const float p0 = fast_exp2(fmaf(s[8 * st + 2 * w], c, -mu));
-        const float p1 = fast_exp2(fmaf(s[8 * st + 2 * w + 1], c, -mu));
-        float h0, h1;
-        if constexpr (IS_BF16) {
-            const bf16x2_t hk = {(__bf16)p0, (__bf16)p1};
-            const uint32_t h = __builtin_bit_cast(uint32_t, hk);
-            h0 = __builtin_bit_cast(float, h << 16);
-            h1 = __builtin_bit_cast(float, h & 0xffff0000u);
-            const bf16x2_t lk = {(__bf16)(p0 - h0), (__bf16)(p1 - h1)};
-            ph[w] = h;
-            pl[w] = __builtin_bit_cast(uint32_t, lk);
-        } else {
-            const f16x2_t hk = {(_Float16)p0, (_Float16)p1};
-            h0 = (float)hk[0];
-            h1 = (float)hk[1];
-            const f16x2_t lk = {(_Float16)(p0 - h0), (_Float16)(p1 - h1)};
-            ph[w] = __builtin_bit_cast(uint32_t, hk);
-            pl[w] = __builtin_bit_cast(uint32_t, lk);
-        }
-        acc[w & 1] += p0 + p1;
-    }
 }
 
 template <int NKB>
@@ -614,6 +574,7 @@ __global__ void __launch_bounds__(64) mfa_combine_kernel(KArgs a) {
     const int b = unit / a.Hq, hq = unit - b * a.Hq;
     const SeqView sv = seq_view<2>(a, b, hq);
     if (qrow >= sv.Lq) return;
+    if (a.single_rows && sv.Lq == 1) return;  // (the single-row kernel stores it)
     const int ns = min(a.nsplit, max(1, (sv.Lk + a.split_keys - 1) / a.split_keys));
     const int64_t stride = (int64_t)a.U * a.Lq;
     float m = -INFINITY;
@@ -664,15 +625,11 @@ __global__ void __launch_bounds__(64) mfa_combine_kernel(KArgs a) {
 //   DP  : head dim padded to a multiple of 32 (32, 64, 96, 128)
 //   QB  : 32-query column blocks per wavefront (workgroup rows = 4*32*QB)
 //   NKB : 32-key row blocks per K/V block (keys per block = 32*NKB)
-//   EXACT: the exact-row instantiation (block_exact below): the kernel of
-//          single-row sequences and packed grouped-query decode rows.  It is
-//          a separate kernel, not a path of the others: a second block path
-//          inside their key loop made the register allocator spill in it.
 // With QB >= 2, unmasked blocks run software-pipelined: the QK^T MFMAs of
 // query block qb+1 and the PV MFMAs of query block qb-1 are interleaved with
 // the softmax VALU work of query block qb, so the matrix cores and the
 // vector ALU run concurrently within one wavefront.
-template <int DP, int QB, int NKB, bool IS_BF16, bool BIAS, bool PAGED, bool EXACT>
+template <int DP, int QB, int NKB, bool IS_BF16, bool BIAS, bool PAGED>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MFA_WAVES_PER_EU)))
 mfa_fwd16_kernel(KArgs a) {
     constexpr int BM = kWaves * QB * 32;
@@ -687,13 +644,7 @@ mfa_fwd16_kernel(KArgs a) {
     constexpr int V_ELEMS = BN * VST;
     constexpr int KV_ELEMS = 2 * (K_ELEMS + V_ELEMS);
     constexpr int Q_ELEMS = BM * KST;
-    // The exact-row kernel's LDS is sized (at least 60 KB) so that two
-    // workgroups share a CU, as with the other kernels' tiles: its decode
-    // workgroups are HBM-streaming, and three per CU at head dim 64 (what
-    // its registers and 43 KB of K/V stages would allow) measured 18% slower
-    // than two (B=64 H=16 Lk=4096 D=64 single rows: 0.238 against 0.201 ms).
-    constexpr int SMEM_KV = KV_ELEMS > Q_ELEMS ? KV_ELEMS : Q_ELEMS;
-    constexpr int SMEM = (EXACT && SMEM_KV < 30000) ? 30000 : SMEM_KV;
+    constexpr int SMEM = KV_ELEMS > Q_ELEMS ? KV_ELEMS : Q_ELEMS;
     constexpr int CPR = DP / 8;                                 // 16-byte chunks per row
     constexpr int KCH = (BN * CPR + kThreads - 1) / kThreads;  // chunks per thread per tile
     typedef typename std::conditional<IS_BF16, bf16x8_t, f16x8_t>::type op_t;
@@ -714,13 +665,11 @@ mfa_fwd16_kernel(KArgs a) {
     // w / (kWaves / R) at position block w % (kWaves / R), so it still holds
     // QB * 32 aligned positions of one head and its rows' arithmetic equals
     // the unpacked tile's.
-    const int hpk = EXACT ? 1 : a.hpack;
+    const int hpk = a.hpack;
     const int PM = BM / hpk;  // positions per tile
     const int q0 = tile * PM;
     if (q0 >= sv.Lq) return;
-    // a varlen call mixing single-row sequences with longer ones: the
-    // exact-row kernel's launch takes the single-row ones, this one the rest
-    if (a.single_rows != 0 && (sv.Lq == 1) != EXACT) return;
+    if (a.single_rows && sv.Lq == 1) return;  // (the single-row kernel's launch computes it)
     // split-KV: this sequence's chunks (one when it has no key)
     if (a.nsplit > 1 && split >= max(1, (sv.Lk + a.split_keys - 1) / a.split_keys)) return;
 
@@ -753,13 +702,7 @@ mfa_fwd16_kernel(KArgs a) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) o[qb][db][r] = 0.f;
     const float c = BIAS ? kLog2e : a.scale_log2;
-    // Exact rows (this instantiation's: single-row sequences and packed
-    // grouped-query decode rows) take per-row rescales -- their results do not
-    // depend on which rows share a wave, so packed heads equal unpacked ones
-    // bit for bit -- and two-term probabilities (block_exact): a single row
-    // averaging thousands of near-equal weights has a small max|O|, against
-    // which one 16-bit rounding of every weight is visible.
-    const float tau = (EXACT || Lq == 1 || a.decode_pack) ? 0.f : (float)MFA_RESCALE_TAU;
+    const float tau = (float)MFA_RESCALE_TAU;
     const float tau_c = tau / c;
 
     // ---- key range of the workgroup and of this wavefront
@@ -951,59 +894,6 @@ mfa_fwd16_kernel(KArgs a) {
         if constexpr (MFA_SIMPLE_PRIO) __builtin_amdgcn_s_setprio(0);
     };
 
-    // Block of the exact-row instantiation: query blocks one at a time, each
-    // skipped when it holds no row of the sequence (a single query row leaves
-    // every block but the wave's first empty), with two-term probabilities
-    // and two PV MFMAs per V fragment (probs16x2_group).
-    auto block_exact = [&](auto masked_tag, const uint16_t* kbuf, const uint16_t* vtb, int j) {
-        constexpr bool MASKED = decltype(masked_tag)::value;
-#pragma unroll
-        for (int qb = 0; qb < QB; ++qb) {
-            if (wq0 + 32 * qb >= Lq) break;  // (wave-uniform)
-            f32x16_t sacc[NKB];
-            if constexpr (MFA_SIMPLE_PRIO) __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-            for (int kb = 0; kb < NKB; ++kb) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) sacc[kb][r] = 0.f;
-#pragma unroll
-                for (int s = 0; s < DS; ++s) {
-                    const op_t kf = *reinterpret_cast<const op_t*>(kbuf + (32 * kb + l32) * KST + 16 * s + 8 * half);
-                    sacc[kb] = mfma16(kf, qf[qb][s], sacc[kb]);
-                }
-            }
-            if constexpr (MFA_SIMPLE_PRIO) __builtin_amdgcn_s_setprio(0);
-            qb_transform<NKB, BIAS, MASKED>(a, sacc, rs[qb], j, half);
-            float alpha;
-            if (qb_update(rs[qb], qb_max<NKB>(sacc), c, tau_c, alpha)) scale_rows<DB>(o[qb], alpha);
-            // each group of 8 weights goes to the PV MFMAs right after it is
-            // formed, so the scores free their registers group by group (the
-            // lo terms would not fit beside all of them at head dim 128);
-            // every O row block still sees the k-steps in the order
-            // (kb, st), hi before lo
-            float acc[2] = {0.f, 0.f};
-#pragma unroll
-            for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-                for (int st = 0; st < 2; ++st) {
-                    // (fenced, so the scheduler does not hoist every group's V
-                    // fragment reads to the top, which would hold them all in
-                    // registers at once)
-                    __builtin_amdgcn_sched_barrier(0);
-                    u32x4_t ph, pl;
-                    probs16x2_group<IS_BF16>(sacc[kb], st, ph, pl, acc, rs[qb].mu, c);
-#pragma unroll
-                    for (int db = 0; db < DB; ++db) {
-                        const op_t vf = load_vf(vtb, db, kb, st);
-                        o[qb][db] = mfma16(vf, __builtin_bit_cast(op_t, ph), o[qb][db]);
-                        o[qb][db] = mfma16(vf, __builtin_bit_cast(op_t, pl), o[qb][db]);
-                    }
-                }
-            __builtin_amdgcn_sched_barrier(0);
-            rs[qb].l += acc[0] + acc[1];
-        }
-    };
-
     // Software-pipelined unmasked block (QB >= 2).  Program order:
     //   QK(0) | QK(1) + softmax(0) | PV(0) + softmax(1) | ... | PV(QB-1)
     // where "+" means the MFMAs are issued one or two at a time between the
@@ -1163,15 +1053,7 @@ mfa_fwd16_kernel(KArgs a) {
         const bool masked = !((j >= w_lo_last) && (j + BN - 1 <= w_hi_first));
         const uint16_t* kbuf = smem + buf * K_ELEMS;
         const uint16_t* vtb = smem + 2 * K_ELEMS + buf * V_ELEMS;  // row-major V
-        if constexpr (EXACT) {
-            if (!skip) {
-                if (masked)
-                    block_exact(std::true_type{}, kbuf, vtb, j);
-                else
-                    block_exact(std::false_type{}, kbuf, vtb, j);
-            }
-            stage_next();
-        } else if (QB >= 2 && MFA_PIPELINE && !skip && !masked) {
+        if (QB >= 2 && MFA_PIPELINE && !skip && !masked) {
             if constexpr (QB >= 2 && MFA_PIPELINE) {
                 if constexpr (MFA_STAGE_IN_PV && MFA_BRANCHFREE_STAGE) {
                     // unconditional staging: no branch splits the pipelined
@@ -1205,7 +1087,7 @@ mfa_fwd16_kernel(KArgs a) {
         store_partial<QB, DB>(a, Lq, b * a.Hq + hq, split, o, rs, c, wq0, lane);
     } else {  // (the loop's last barrier released the LDS)
         SeqView svh = sv;  // this wave's head: its O and lse rows
-        if (!EXACT && hl != 0) {
+        if (hl != 0) {
             svh.o += (int64_t)hl * a.oh1 * (a.out_f32 ? 4 : 2);
             if (svh.lse) svh.lse += (int64_t)hl * a.lse_h1;
         }
@@ -1278,7 +1160,7 @@ mfa_fwd16_pp_kernel(KArgs a) {
     const int PM = BM / hpk;  // positions per tile
     const int q0 = tile * PM;
     if (q0 >= sv.Lq) return;
-    if (a.single_rows != 0 && sv.Lq == 1) return;  // (the exact-row kernel's launch computes it)
+    if (a.single_rows && sv.Lq == 1) return;  // (the single-row kernel's launch computes it)
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
@@ -1765,7 +1647,7 @@ mfa_fwd16_tk_kernel(KArgs a) {
     const SeqView sv = seq_view<2>(a, b, hq);
     const int q0 = tile * BM;
     if (q0 >= sv.Lq) return;
-    if (a.single_rows != 0 && sv.Lq == 1) return;  // (the exact-row kernel's launch computes it)
+    if (a.single_rows && sv.Lq == 1) return;  // (the single-row kernel's launch computes it)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
     const int Lq = sv.Lq, Lk = sv.Lk, D = a.D;
@@ -1852,7 +1734,7 @@ mfa_fwd16_tk_kernel(KArgs a) {
             return __builtin_amdgcn_mfma_f32_32x32x16_f16(x, y, acc, 0, 0, 0);
     };
     const float c = BIAS ? kLog2e : a.scale_log2;
-    const float tau = (Lq == 1 || a.decode_pack) ? 0.f : (float)MFA_RESCALE_TAU;
+    const float tau = (float)MFA_RESCALE_TAU;
     const float tau_c = tau / c;
     const float slope = a.alibi ? a.alibi[b * a.alibi_bstride + hq] : 0.f;
     // a key past the second 16 never carries weight when Lk <= 16: one PV step
@@ -2135,6 +2017,8 @@ int set_err(int code, const char* fmt, ...) {
 }
 
 typedef void (*kernel_fn)(KArgs);
+typedef void (*decode_fn)(DArgs);
+
 
 struct KernelCfg {
     kernel_fn fn;
@@ -2145,24 +2029,13 @@ struct KernelCfg {
     int threads = kThreads;  // threads per workgroup
 };
 
-template <int DP, int QB, int NKB, bool IS_BF16, bool BIAS, bool EXACT = false>
+template <int DP, int QB, int NKB, bool IS_BF16, bool BIAS>
 KernelCfg cfg16(const char* name, bool paged) {
     constexpr int BM = kWaves * QB * 32, BN = NKB * 32;
     constexpr int kv = 2 * (BN * (DP + 8) + BN * (DP + MFA_V_PAD)), qs = BM * (DP + 8);
-    return KernelCfg{paged ? (kernel_fn)mfa_fwd16_kernel<DP, QB, NKB, IS_BF16, BIAS, true, EXACT>
-                           : (kernel_fn)mfa_fwd16_kernel<DP, QB, NKB, IS_BF16, BIAS, false, EXACT>,
+    return KernelCfg{paged ? (kernel_fn)mfa_fwd16_kernel<DP, QB, NKB, IS_BF16, BIAS, true>
+                           : (kernel_fn)mfa_fwd16_kernel<DP, QB, NKB, IS_BF16, BIAS, false>,
                      BM, BN, 2 * (kv > qs ? kv : qs), name};
-}
-// the exact-row kernel: one 32-row query block per wavefront (128-row tiles),
-// 64-key blocks
-template <bool IS_BF16, bool BIAS>
-KernelCfg select16x(int dp, bool paged) {
-    switch (dp) {
-        case 32: return cfg16<32, 1, 2, IS_BF16, BIAS, true>(IS_BF16 ? "mfa_fwd16x<bf16,d32>" : "mfa_fwd16x<f16,d32>", paged);
-        case 64: return cfg16<64, 1, 2, IS_BF16, BIAS, true>(IS_BF16 ? "mfa_fwd16x<bf16,d64>" : "mfa_fwd16x<f16,d64>", paged);
-        case 96: return cfg16<96, 1, 2, IS_BF16, BIAS, true>(IS_BF16 ? "mfa_fwd16x<bf16,d96>" : "mfa_fwd16x<f16,d96>", paged);
-        default: return cfg16<128, 1, 2, IS_BF16, BIAS, true>(IS_BF16 ? "mfa_fwd16x<bf16,d128>" : "mfa_fwd16x<f16,d128>", paged);
-    }
 }
 template <int DP, int QB, int NKB, bool IS_BF16, bool BIAS, int NW = 8>
 KernelCfg cfg16pp(const char* name) {
@@ -2279,20 +2152,22 @@ struct Plan {
     bool empty;
     kernel_fn combine = nullptr;  // split-KV merge kernel
     int64_t ws_bytes = 0;         // split-KV workspace
-    // second launch (after the first, before a split-KV merge): the exact-row
-    // kernel on the single-row sequences of a varlen call that mixes them
-    // with longer ones
-    bool second = false;
-    KernelCfg cfg2;
-    KArgs args2;
-    int grid2 = 0;
+    // the single-row kernel: instead of the above (decode_only: every sequence
+    // of the call has one query row; combine is then its merge kernel, for
+    // dec.nsplit > 1), or as a second launch on the single-row sequences of a
+    // varlen call that mixes them with longer ones
+    bool decode_only = false, decode_too = false;
+    DecodeKernels dk;
+    DArgs dec;
+    int dec_grid = 0;
 };
 
 // Enqueue a plan's kernel launches (the split-KV merge aside).
 void launch_plan(const Plan& plan, hipStream_t st) {
-    hipLaunchKernelGGL(plan.cfg.fn, dim3(plan.grid), dim3(plan.cfg.threads), 0, st, plan.args);
-    if (plan.second)
-        hipLaunchKernelGGL(plan.cfg2.fn, dim3(plan.grid2), dim3(plan.cfg2.threads), 0, st, plan.args2);
+    if (!plan.decode_only)
+        hipLaunchKernelGGL(plan.cfg.fn, dim3(plan.grid), dim3(plan.cfg.threads), 0, st, plan.args);
+    if (plan.decode_only || plan.decode_too)
+        hipLaunchKernelGGL((decode_fn)plan.dk.attend, dim3(plan.dec_grid), dim3(kDecodeThreads), 0, st, plan.dec);
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -2392,36 +2267,87 @@ ChipGeom chip_geometry_of(hipStream_t st) {
 }
 ChipGeom chip_geometry_current() { return chip_geometry_of(nullptr); }
 
+// Chunks per workgroup of a single-row call (>= nmax: a workgroup walks all of
+// its unit's, and no merge runs).  One, until every CU has two workgroups, then
+// two: longer walks save little more and leave CUs idle at the end.  A walk of
+// the whole unit saves the partial results and the merge (its launch is about 4
+// us, a chunk in a walk 2.5), and wins for at most two chunks and in dense calls
+// whose units come out close to whole rounds of one per CU (at head dims up to
+// 64, where a CU takes more of them at once, from two per CU); ragged sequences
+// end too far apart.  Measured (bf16, us per call; chunks per workgroup 1 / 2 / 4 /
+// all; Hq=32 Hkv=8 D=128 where not said):
+//   B=1 Lk=3001 (8 units)                 12.0 / 14.6 / 20.3 / 38.0
+//   B=1 Lk=512 D=64                        7.7 /  6.6 (all)
+//   B=8 Lk=4096 (64 units)                35.7 / 36.5 / 35.2 / 67.9
+//   B=16 (128)                            61.8 / 59.9 / 58.1 / 72.4
+//   B=24 (192)                            89.5 / 87.6 / 86.0 / 82.2
+//   B=32 (256)                           114.5 / 111.6 / 110.3 / 97.6
+//   B=33 (264)                           121.1 / 117.8 / 121.8 / 141.4
+//   B=48 (384)                           173.5 / 165.5 / 163.3 / 159.3
+//   B=1 Lk=128K H=16 (16)                191.1 / 192.1 / 189.8 / 1470
+//   B=48 Lk=6000 Hq=32 Hkv=4 D=64 (192)   65.8 / 67.4 / 70.0 / 78.7
+//   B=64 Lk=4096 H=16 D=64 (1024)        215.1 / 218.3 / 218.2 / 201.2
+//   varlen, lengths uniform in [max/16, max]:
+//   24 sequences to 4096 (192)            56.7 / 56.0 / 60.7 / 70.2
+//   64 to 4096 (512)                     138.5 / 134.0 / 136.2 / 140.2
+//   48 to 8192, H=16 D=64 (768)          185.9 / 187.3 / 190.2 / 212.7
+int64_t decode_group(int64_t units, int64_t nmax, int dp, bool varlen, int cus) {
+    const int64_t rounds = (units + cus - 1) / cus;
+    const bool fills = dp > 64 ? 4 * units >= 3 * cus * rounds : units >= 2 * (int64_t)cus;
+    if (nmax <= 2 || (!varlen && fills)) return nmax;
+    return units * nmax <= 2 * (int64_t)cus ? 1 : 2;
+}
+KernelCfg single_cfg(int dp, bool bf16, int lds) {
+    static const char* const names[2][4] = {
+        {"mfa_fwd16x<f16,d32>", "mfa_fwd16x<f16,d64>", "mfa_fwd16x<f16,d96>", "mfa_fwd16x<f16,d128>"},
+        {"mfa_fwd16x<bf16,d32>", "mfa_fwd16x<bf16,d64>", "mfa_fwd16x<bf16,d96>", "mfa_fwd16x<bf16,d128>"}};
+    return KernelCfg{nullptr, kDecodeRows, 128, lds, names[bf16][dp / 32 - 1], kDecodeThreads};
+}
+
+// The single-row kernel's launch for the call in plan->args: every (sequence,
+// K/V head, up to 16 of its query heads), walking the chunks of its keys in
+// one workgroup or, with `may_split` (the call has a workspace) and where that
+// is faster, in several.  The results are the same bits either way.
+int plan_decode(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int dp, bool bias, bool may_split) {
+    DArgs& d = plan->dec;
+    memset(&d, 0, sizeof(d));
+    d.f = plan->args;
+    d.R = p->heads_q / p->heads_kv;
+    d.rt = (d.R + kDecodeRows - 1) / kDecodeRows;
+    d.nr = std::min(d.R, kDecodeRows);
+    const int64_t units = (int64_t)p->batch * p->heads_kv * d.rt;
+    if (units > 0x7fffffffLL / 2 || (int64_t)p->batch * p->heads_q > 0x7fffffffLL / 2)
+        return set_err(MFA_ERR_INVALID, "mfa_fwd: problem too large");
+    d.units = (int32_t)units;
+    d.nsplit = 1;
+    d.group = INT32_MAX / 2;
+    d.bias = bias;
+    // Every K/V row is read once, by one workgroup (two above 16 heads per K/V
+    // head): non-temporal loads, where K and V are too large to be still in the
+    // caches from when they were written (us, plain -> non-temporal: B=64
+    // Lk=4096 Hq=32 Hkv=8 D=128, 1 GB, 187.4 -> 167.1; B=8, 134 MB, 35.9 ->
+    // 30.5; 48 ragged sequences to 8192, H=16 D=64, 185.3 -> 164.1; but B=6
+    // Lk=1500 H=16 D=64, 37 MB, 14.4 -> 15.4).
+    d.nt = (int64_t)p->batch * p->seqlen_k * p->heads_kv * p->head_dim * 4 >= ((int64_t)64 << 20) && d.rt <= 2;
+    d.ws_ld = dp;
+    plan->ws_bytes = 0;
+    const int64_t nmax = decode_chunks_max(p->seqlen_k);
+    if (may_split && nmax > 1) {
+        const int64_t rows = nmax * units * d.nr;
+        const int64_t group = decode_group(units, nmax, dp, p->cu_seqlens_q != nullptr, geom.cus);
+        if (group < nmax && units * nmax <= 0x7fffffffLL / 2 && rows <= 0x7fffffffLL / 2) {
+            d.group = (int32_t)group;
+            d.nsplit = (int32_t)((nmax + group - 1) / group);
+            plan->ws_bytes = rows * dp * 4 + (rows * 8 + 255) / 256 * 256;
+        }
+    }
+    plan->dec_grid = (int)(units * d.nsplit);
+    plan->dk = mfa_decode_kernels(dp, p->dtype_in == MFA_DTYPE_BF16, p->block_table != nullptr);
+    return MFA_OK;
+}
+
 int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int split_keys = 0) {
     if (!p) return set_err(MFA_ERR_INVALID, "mfa_fwd: params is NULL");
-    // Single-row grouped-query decode: the R query heads of a K/V head become
-    // the R rows of one sequence (the same q/o memory through other strides),
-    // so one workgroup reads each K/V head once for all of them.  Exact for
-    // rows whose valid keys do not depend on their position -- no window, no
-    // ALiBi; causal with one query row admits every key -- and, with the
-    // per-row rescales of such rows, bit-identical to the unpacked call.
-    // Varlen calls whose longest query is one row pack the same way (a
-    // sequence's rows are its one token's query heads); there the lse rows
-    // of one token would not be contiguous, so only without an lse output.
-    const int64_t tok_qs = p->q_seq_stride, tok_os = p->o_seq_stride;  // token strides (varlen starts)
-    mfa_fwd_params packed;
-    bool pack = false;
-    const bool lse_ok = p->cu_seqlens_q ? !p->softmax_lse : (!p->softmax_lse || p->lse_head_stride == 1);
-    if (p->dtype_in != MFA_DTYPE_F32 && p->seqlen_q == 1 && p->heads_kv > 0 && p->heads_q > p->heads_kv &&
-        p->heads_q % p->heads_kv == 0 && p->window_left < 0 && p->window_right < 0 && !p->alibi_slopes && lse_ok) {
-        const int R = p->heads_q / p->heads_kv;
-        packed = *p;
-        packed.seqlen_q = R;
-        packed.heads_q = p->heads_kv;
-        packed.q_seq_stride = p->q_head_stride;
-        packed.q_head_stride = p->q_head_stride * R;
-        packed.o_seq_stride = p->o_head_stride;
-        packed.o_head_stride = p->o_head_stride * R;
-        packed.causal = 0;
-        if (p->softmax_lse) packed.lse_head_stride = R;
-        p = &packed;
-        pack = true;
-    }
     const int din = p->dtype_in, dout = p->dtype_out;
     if (din != MFA_DTYPE_F16 && din != MFA_DTYPE_BF16 && din != MFA_DTYPE_F32)
         return set_err(MFA_ERR_INVALID, "mfa_fwd: unknown dtype_in %d", din);
@@ -2641,30 +2567,24 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
         else
             pp256 = prefer_pp256(p, geom.cus);
     }
-    // Exact rows: a 16-bit call whose every sequence has one query row, or a
-    // packed grouped-query decode, runs the exact-row kernel (two-term
-    // probabilities, per-row rescales), whatever the tile hint.  A varlen
-    // call that may mix single-row sequences with longer ones runs its kernel
-    // on the longer ones and the exact-row kernel on the single-row ones
-    // (a second launch, planned below), so each sequence's rows are those of
-    // its own dense call.
-    const bool exact_call = din != MFA_DTYPE_F32 && (pack || p->seqlen_q == 1);
+    // Single rows: a 16-bit call whose every sequence has one query row runs
+    // the single-row kernel, whatever the tile hint.  A varlen call that may
+    // mix such sequences with longer ones runs its kernel on the longer ones
+    // and the single-row kernel on the others (a second launch), so each
+    // sequence's rows are those of its own dense call.
+    const bool single_call = din != MFA_DTYPE_F32 && p->seqlen_q == 1;
     const bool mixed_rows =
-        din != MFA_DTYPE_F32 && !exact_call && p->cu_seqlens_q != nullptr && !p->varlen_no_single_rows;
+        din != MFA_DTYPE_F32 && !single_call && p->cu_seqlens_q != nullptr && !p->varlen_no_single_rows;
     // At most 32 keys per sequence under many query rows (cross-attention to
     // a short conditioning sequence): the tiny-key kernel, which keeps the
     // keys in registers and streams the query rows (measured at bf16 D=128
     // Lq=26136 Lk=5 H=16: see the design notes)
     const bool tiny_keys = MFA_TK && p->tile_hint == MFA_TILE_AUTO && din != MFA_DTYPE_F32 && !paged &&
-                           !exact_call && split_keys == 0 && p->seqlen_k <= 32 && p->seqlen_q >= MFA_TK_MIN_ROWS;
-    auto exact_cfg = [&]() {
-        if (din == MFA_DTYPE_BF16) return bias ? select16x<true, true>(dp, paged) : select16x<true, false>(dp, paged);
-        return bias ? select16x<false, true>(dp, paged) : select16x<false, false>(dp, paged);
-    };
+                           !single_call && split_keys == 0 && p->seqlen_k <= 32 && p->seqlen_q >= MFA_TK_MIN_ROWS;
     if (din == MFA_DTYPE_F32)
         plan->cfg = bias ? select32<true>(dp, paged) : select32<false>(dp, paged);
-    else if (exact_call)
-        plan->cfg = exact_cfg();
+    else if (single_call)
+        plan->cfg = single_cfg(dp, din == MFA_DTYPE_BF16, 0);  // (its LDS is plan_decode's choice)
     else if (tiny_keys && din == MFA_DTYPE_BF16)
         plan->cfg = bias ? select16tk<true, true>(dp) : select16tk<true, false>(dp);
     else if (tiny_keys)
@@ -2702,10 +2622,6 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
     a.wl = p->window_left < 0 ? -1 : (int32_t)(p->window_left > wmax ? wmax : p->window_left);
     a.wr = p->window_right < 0 ? -1 : (int32_t)(p->window_right > wmax ? wmax : p->window_right);
     a.causal = p->causal ? 1 : 0;
-    a.decode_pack = pack ? 1 : 0;
-    a.qts = tok_qs;
-    a.ots = tok_os;
-    a.pack_r = (pack && p->cu_seqlens_q) ? p->seqlen_q : 1;  // packed varlen: R rows per query token
     a.single_rows = mixed_rows ? 1 : 0;
     a.out_f32 = dout == MFA_DTYPE_F32 ? 1 : 0;
     a.lse = p->softmax_lse;
@@ -2733,6 +2649,23 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
         a.bt_b = 0;
     }
 
+    plan->decode_only = plan->decode_too = false;
+    if (split_keys != 0 && (p->seqlen_k + (int64_t)split_keys - 1) / split_keys > kMaxSplits)
+        return set_err(MFA_ERR_INVALID, "mfa_fwd_splitkv: %d chunks of %d keys exceed %d; use larger chunks",
+                       (int)((p->seqlen_k + (int64_t)split_keys - 1) / split_keys), split_keys, kMaxSplits);
+    if (single_call || mixed_rows) {
+        const int rc = plan_decode(p, plan, geom, dp, bias, split_keys != 0 && single_call);
+        if (rc != MFA_OK) return rc;
+        if (single_call) {
+            plan->decode_only = true;
+            plan->grid = plan->dec_grid;
+            plan->cfg.lds = plan->dk.lds;
+            if (plan->grid == 0) plan->empty = true;
+            return MFA_OK;
+        }
+        plan->decode_too = !plan->empty && plan->dec_grid > 0;
+    }
+
     // Ping-pong tiles of a grouped-query call with 2, 4 or 8 query heads per
     // K/V head pack those heads into one tile (KArgs.hpack): each head takes
     // 1/R of the tile's rows at the same positions, so a tile streams its K/V
@@ -2749,7 +2682,7 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
     // The 4-wavefront 16-bit kernel packs 2 or 4 heads the same way (one or
     // two wavefronts per head), except for split-KV and paged calls.
     const bool pack_pp = MFA_PP_HEAD_PACK && plan->cfg.threads == 8 * 64 && (R == 2 || R == 4 || R == 8);
-    const bool pack_4w = MFA_4W_HEAD_PACK && din != MFA_DTYPE_F32 && !exact_call && !tiny_keys && !paged &&
+    const bool pack_4w = MFA_4W_HEAD_PACK && din != MFA_DTYPE_F32 && !tiny_keys && !paged &&
                          split_keys == 0 && plan->cfg.threads == kThreads && (R == 2 || R == 4);
     if (pack_pp || pack_4w) {
         a.hpack = R;
@@ -2791,9 +2724,6 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
     a.nsplit = 1;
     if (split_keys != 0) {
         const int ns = (p->seqlen_k + split_keys - 1) / split_keys;
-        if (ns > kMaxSplits)
-            return set_err(MFA_ERR_INVALID, "mfa_fwd_splitkv: %d chunks of %d keys exceed %d; use larger chunks", ns,
-                           split_keys, kMaxSplits);
         a.nsplit = ns > 1 ? ns : 1;
         a.split_keys = split_keys;
         a.ws_ld = dp;
@@ -2807,26 +2737,6 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
         plan->combine = din == MFA_DTYPE_BF16 ? (kernel_fn)mfa_combine_kernel<true> : (kernel_fn)mfa_combine_kernel<false>;
     }
     if (plan->grid == 0) plan->empty = true;
-    plan->second = false;
-    if (mixed_rows && !plan->empty) {
-        // the exact-row kernel over one query tile (times the split chunks)
-        // of every (sequence, head); it computes the single-row sequences only
-        plan->second = true;
-        plan->cfg2 = exact_cfg();
-        KArgs& a2 = plan->args2;
-        a2 = a;
-        a2.single_rows = 2;
-        // (one head per unit: undo a head-packed main launch's strides)
-        a2.hpack = 1;
-        a2.Hq = p->heads_q;
-        a2.qh = a.qh1;
-        a2.oh = a.oh1;
-        a2.lse_h = a.lse_h1;
-        a2.U = p->batch * p->heads_q;
-        a2.upx = a.grouped ? (int32_t)(G / X) * R : 0;
-        a2.T = a.nsplit;
-        plan->grid2 = (a.grouped ? X * a2.upx : a2.U) * a2.T;
-    }
     return MFA_OK;
 }
 
@@ -2855,14 +2765,21 @@ int auto_split_keys(const mfa_fwd_params* p, const ChipGeom& geom) {
 // kernel reads (each chunk of each row that exists, lse -inf and O 0 for a
 // chunk without a valid key), so the workspace needs no clearing.
 int launch_splitkv(Plan& plan, void* ws, hipStream_t st, const char* who) {
+    if (plan.decode_only) {
+        DArgs& d = plan.dec;
+        d.ws_o = static_cast<float*>(ws);
+        d.ws_ml = d.ws_o + (int64_t)decode_chunks_max(d.f.Lk) * d.units * d.nr * d.ws_ld;
+        launch_plan(plan, st);
+        if (d.nsplit > 1)
+            hipLaunchKernelGGL((decode_fn)plan.dk.merge, dim3((unsigned)(d.units * d.nr)), dim3(64), 0, st, d);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return set_err(MFA_ERR_LAUNCH, "%s: launch failed: %s", who, hipGetErrorString(e));
+        return MFA_OK;
+    }
     KArgs& a = plan.args;
-    // (the planned rows: a packed grouped-query decode has a.Lq = query heads
-    // per K/V head rows per unit, not the caller's seqlen_q)
     const int64_t rows = (int64_t)a.nsplit * a.U * a.Lq;
     a.ws_o = static_cast<float*>(ws);
     a.ws_lse = a.ws_o + rows * a.ws_ld;
-    plan.args2.ws_o = a.ws_o;
-    plan.args2.ws_lse = a.ws_lse;
     // one chunk (every key range fits): the kernels store O themselves
     launch_plan(plan, st);
     if (a.nsplit > 1)
@@ -2985,11 +2902,24 @@ int mfa_fwd_splitkv_static(const mfa_fwd_params* params, int32_t split_keys, voi
     const int rc = make_plan(params, &plan, chip_geometry_of(static_cast<hipStream_t>(stream)), split_keys);
     if (rc != MFA_OK) return rc;
     if (plan.empty) return MFA_OK;
-    if (plan.ws_bytes > MFA_STATIC_SCRATCH_BYTES)
+    int64_t need = plan.ws_bytes;
+    if (plan.decode_only) {
+        // single rows: the size of the request's own chunks decides whether
+        // the call is taken; beyond the scratch, a workgroup walks the chunks
+        const mfa_fwd_params* p = params;
+        const int64_t rows = ((int64_t)p->seqlen_k + split_keys - 1) / split_keys * p->batch * p->heads_q;
+        if (need > MFA_STATIC_SCRATCH_BYTES) {
+            plan.dec.nsplit = 1;
+            plan.dec.group = INT32_MAX / 2;
+            plan.dec_grid = plan.dec.units;
+        }
+        need = rows * plan.dec.ws_ld * 4 + (rows * 4 + 255) / 256 * 256;
+    }
+    if (need > MFA_STATIC_SCRATCH_BYTES)
         return set_err(MFA_ERR_INVALID,
                        "mfa_fwd_splitkv_static: this call needs %lld bytes of workspace, more than the static "
                        "scratch's %lld; use mfa_fwd_splitkv with a caller workspace, or larger chunks",
-                       (long long)plan.ws_bytes, (long long)MFA_STATIC_SCRATCH_BYTES);
+                       (long long)need, (long long)MFA_STATIC_SCRATCH_BYTES);
     const hipStream_t st = static_cast<hipStream_t>(stream);
     void* ws = nullptr;
     const int src = static_scratch(st, &ws);
