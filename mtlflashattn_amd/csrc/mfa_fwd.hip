@@ -62,6 +62,7 @@
 #include "mfa.h"
 #include "mfa_common.h"
 #include "mfa_decode.h"
+#include "mfa_tile32.h"
 
 namespace {
 
@@ -1813,7 +1814,8 @@ mfa_fwd16_tk_kernel(KArgs a) {
 }
 
 // ----------------------------------------------------------------------------
-// fp32 kernel: same structure with v_mfma_f32_32x32x2_f32.  K-slot layout of
+// fp32 kernel: same structure with v_mfma_f32_32x32x2_f32 (grids that fill the
+// chip; mfa_fwd32s_kernel below serves the others).  K-slot layout of
 // the 32x32x2 MFMA: lane (half, x) supplies k = half, so QK^T step s uses
 // d = s + half*DP/2 and PV step r uses the key held in accumulator register r.
 template <int DP, int NKB, bool BIAS, bool PAGED>
@@ -2004,6 +2006,155 @@ __global__ void __launch_bounds__(kThreads) mfa_fwd32_kernel(KArgs a) {
 }
 
 // ----------------------------------------------------------------------------
+// fp32 kernel (v_mfma_f32_32x32x2_f32): 32 query rows per workgroup (lane =
+// query, as in the 16-bit kernels), NW wavefronts that take every NW-th 32-key
+// block, each with its own K and V tile in LDS and its own running softmax, no
+// barrier until their states are merged at the end.  Bound by the matrix pipe:
+// a 32 x 32 block is DP MFMAs of 64 cycles against ~250 vector instructions,
+// and re-reading K/V for every 32 rows costs 4 bytes per cycle and wavefront.
+// The split over keys rather than rows is for the grids and walks: 128-row
+// workgroups of mfa_fwd32_kernel leave most CUs idle on short sequences and
+// walk every key in each.  A tile's loads go straight to LDS as
+// soon as its last reader is done: the next K behind the softmax and PV, the
+// next V behind the next QK.  prefer_split32 has the measurements and the rule.
+template <int DP, int NW, bool BIAS, bool PAGED>
+__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(DP <= 64 ? 2 : 1)))
+mfa_fwd32s_kernel(KArgs a) {
+    typedef Tile<DP> T;
+    constexpr int DB = DP / 32, BM = 32, BN = 32;
+    __shared__ __attribute__((aligned(16))) float k_s[NW][T::FLOATS];
+    __shared__ __attribute__((aligned(16))) float v_s[NW][T::FLOATS];
+    __shared__ float m_s[NW][BM], l_s[NW][BM];
+
+    int b, hq, tile;
+    if (!decode_tile(a, blockIdx.x, b, hq, tile)) return;
+    const SeqView sv = seq_view<4>(a, b, hq);
+    const int q0 = tile * BM;
+    if (q0 >= sv.Lq) return;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int Lq = sv.Lq, Lk = sv.Lk, D = a.D;
+    const int dq = Lk - Lq;
+    const int row = q0 + l32, nrow = min(BM, Lq - q0);
+    float* kt = k_s[wave];
+    float* vt = v_s[wave];
+
+    // key blocks any row of the tile sees; this wavefront's are wave, wave + NW, ...
+    const int klo = key_lo(a, q0 + dq), khi = key_hi(a, q0 + nrow - 1 + dq, Lk);
+    const int jbeg = (klo / BN) * BN;
+    const int nblk = khi >= klo ? (khi - jbeg) / BN + 1 : 0;
+    auto load_k = [&](int it) {
+        const int j = jbeg + BN * it;
+        bool ok;
+        const int64_t off = kv_block_off<PAGED>(a, sv, j, Lk, a.kb, a.ks, ok);
+        T::load(kt, reinterpret_cast<const float*>(sv.k) + off, a.ks, ok ? min(BN, Lk - j) : 0, D, lane, false);
+    };
+    auto load_v = [&](int it) {
+        const int j = jbeg + BN * it;
+        bool ok;
+        const int64_t off = kv_block_off<PAGED>(a, sv, j, Lk, a.vb, a.vs, ok);
+        T::load(vt, reinterpret_cast<const float*>(sv.v) + off, a.vs, ok ? min(BN, Lk - j) : 0, D, lane, false);
+    };
+    if (wave < nblk) {
+        load_k(wave);
+        load_v(wave);
+    }
+    float qf[DP / 2];
+    row_operand<DP>(qf, reinterpret_cast<const float*>(sv.q) + (int64_t)row * a.qs, row < Lq, D, half);
+    RowState rs;
+    rs.center = row + dq;
+    rs.lo = key_lo(a, rs.center);
+    rs.hi = key_hi(a, rs.center, Lk);
+    rs.slope = a.alibi ? a.alibi[b * a.alibi_bstride + hq] : 0.f;
+    row_reset(rs);
+#pragma unroll
+    for (int s = 0; s < DP / 2; ++s) pin(qf[s]);  // (waited for here: a wait in the loop would drain the tiles' loads)
+    pin(rs.slope);
+    int off[4];
+    T::col_offsets(off, l32, half);
+    f32x16_t o[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
+    const float c = BIAS ? kLog2e : a.scale_log2;
+    const float tau_c = (float)MFA_RESCALE_TAU / c;
+    const int lo_last = key_lo(a, q0 + nrow - 1 + dq), hi_first = key_hi(a, q0 + dq, Lk);
+
+    for (int it = wave; it < nblk; it += NW) {
+        const bool more = it + NW < nblk;
+        const int j = jbeg + BN * it;
+        f32x16_t s[1];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[0][r] = 0.f;
+        wait_vm<T::N>();  // (K's loads were issued before V's)
+        T::rows_product(kt, qf, l32, half, s[0]);
+        wait_lds();
+        if (more) load_k(it + NW);
+        if (j >= lo_last && j + BN - 1 <= hi_first)
+            qb_transform<1, BIAS, false, true>(a, s, rs, j, half);
+        else
+            qb_transform<1, BIAS, true, true>(a, s, rs, j, half);
+        float alpha;
+        if (qb_update(rs, qb_max<1>(s), c, tau_c, alpha)) scale_rows<DB>(o, alpha);
+        qb_probs32<1>(s, rs.l, rs.mu, c);
+        if (more)
+            wait_vm<T::N>();
+        else
+            wait_vm<0>();
+        T::cols_product(vt, off, s[0], o);
+        wait_lds();
+        if (more) load_v(it + NW);
+    }
+
+    // the wavefronts' states: O through the V tiles, exponent reference and sum
+    T::put(vt, o, l32, half);
+    const float lsum = sum_halves(rs.l);
+    if (half == 0) {
+        m_s[wave][l32] = rs.m == -INFINITY ? -INFINITY : rs.mu;
+        l_s[wave][l32] = lsum;
+    }
+    __syncthreads();
+    for (int cc = tid; cc < BM * T::CPR; cc += NW * 64) {
+        const int r = cc / T::CPR, col = ((cc % T::CPR) ^ T::swz(r)) * 4;
+        if (r >= nrow) continue;
+        float m = m_s[0][r];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) m = fmax_nn(m, m_s[w][r]);
+        float x[4] = {0.f, 0.f, 0.f, 0.f}, l = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float mw = m_s[w][r], e = mw == -INFINITY ? 0.f : fast_exp2(mw - m);
+            const float4 y = *reinterpret_cast<const float4*>(v_s[w] + cc * 4);
+            x[0] = fmaf(y.x, e, x[0]);
+            x[1] = fmaf(y.y, e, x[1]);
+            x[2] = fmaf(y.z, e, x[2]);
+            x[3] = fmaf(y.w, e, x[3]);
+            l = fmaf(l_s[w][r], e, l);
+        }
+        const float inv = l > 0.f ? 1.f / l : 0.f;
+        typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4v_t;
+        if (col < D)
+            store_stream(reinterpret_cast<f32x4v_t*>(reinterpret_cast<float*>(sv.o) + (int64_t)(q0 + r) * a.os + col),
+                         f32x4v_t{x[0] * inv, x[1] * inv, x[2] * inv, x[3] * inv});
+        if (sv.lse && col == 0) {
+            float lse = l > 0.f ? (m + __builtin_amdgcn_logf(l)) * kLn2 : -INFINITY;
+            if constexpr (BIAS) {
+                // the lse of the unshifted ALiBi scores (qb_transform's PRECISE form)
+                if (a.alibi) {
+                    RowState t;
+                    t.center = q0 + r + dq;
+                    t.lo = key_lo(a, t.center);
+                    t.hi = key_hi(a, t.center, Lk);
+                    lse -= rs.slope * (float)row_dmin(t);
+                }
+            }
+            sv.lse[q0 + r] = lse;
+        }
+    }
+}
+
+// ----------------------------------------------------------------------------
 // host side
 
 thread_local char g_err[512] = "";
@@ -2065,6 +2216,14 @@ KernelCfg cfg32(const char* name, bool paged) {
     return KernelCfg{paged ? (kernel_fn)mfa_fwd32_kernel<DP, NKB, BIAS, true>
                            : (kernel_fn)mfa_fwd32_kernel<DP, NKB, BIAS, false>,
                      BM, BN, 4 * (kv > qs ? kv : qs), name};
+}
+
+template <int DP, bool BIAS>
+KernelCfg cfg32s(const char* name, bool paged) {
+    constexpr int NW = DP <= 64 ? 8 : 4;  // (what 160 KB of LDS hold)
+    return KernelCfg{paged ? (kernel_fn)mfa_fwd32s_kernel<DP, NW, BIAS, true>
+                           : (kernel_fn)mfa_fwd32s_kernel<DP, NW, BIAS, false>,
+                     32, 32, NW * (2 * 32 * DP + 64) * 4, name, NW * 64};
 }
 
 // tile configuration per (dtype, padded head dim, bias)
@@ -2136,7 +2295,15 @@ KernelCfg select16(int dp, bool fills_chip, bool paged, bool pp256) {
     }
 }
 template <bool BIAS>
-KernelCfg select32(int dp, bool paged) {
+KernelCfg select32(int dp, bool split, bool paged) {
+    if (split) {
+        switch (dp) {
+            case 32: return cfg32s<32, BIAS>("mfa_fwd32<f32,d32,q32,k32,split>", paged);
+            case 64: return cfg32s<64, BIAS>("mfa_fwd32<f32,d64,q32,k32,split>", paged);
+            case 96: return cfg32s<96, BIAS>("mfa_fwd32<f32,d96,q32,k32,split>", paged);
+            default: return cfg32s<128, BIAS>("mfa_fwd32<f32,d128,q32,k32,split>", paged);
+        }
+    }
     switch (dp) {
         case 32: return cfg32<32, 1, BIAS>("mfa_fwd32<f32,d32,q32,k32>", paged);
         case 64: return cfg32<64, 1, BIAS>("mfa_fwd32<f32,d64,q32,k32>", paged);
@@ -2297,6 +2464,37 @@ int64_t decode_group(int64_t units, int64_t nmax, int dp, bool varlen, int cus) 
     if (nmax <= 2 || (!varlen && fills)) return nmax;
     return units * nmax <= 2 * (int64_t)cus ? 1 : 2;
 }
+// fp32: the key-split kernel (32-row workgroups) or the 128-row one.  The
+// 128-row tiles are cheaper per pair where they fill the chip, but come in few
+// and unequal pieces: their time is estimated as whole rounds of one tile per CU
+// (equal tiles) or max(heaviest tile, total / CUs), the split's as total / CUs
+// over 32-row tiles times 1.2 (1.3 above head dim 64, where its LDS leaves one
+// wavefront per SIMD).  Measured (us, 128-row -> split): D=64 B=1 L=512 H=2 48.4
+// -> 15.2, B=2 L=1024 H=8 causal 89.8 -> 34.1, B=3 L=1024 H=16 187 -> 145, but
+// B=32 L=200 H=8 56.0 -> 65.9; D=128 B=2 L=1024 H=16 causal 159 -> 122, B=1
+// L=3000 H=16 892 -> 807, but B=3 L=1024 H=16 causal 160 -> 182 and B=4 L=2000
+// H=8 613 -> 736.
+bool prefer_split32(const mfa_fwd_params* p, int dp, int cus) {
+    if (p->seqlen_q > (1 << 14)) return false;  // (bounds the loops; long rows fill the chip)
+    const int64_t dq = (int64_t)p->seqlen_k - p->seqlen_q;
+    int64_t heaviest = 0, total[2] = {0, 0}, tiles[2] = {0, 0};
+    for (int k = 0; k < 2; ++k) {
+        const int rows = k ? 32 : 128;
+        for (int64_t r0 = 0; r0 < p->seqlen_q; r0 += rows, ++tiles[k]) {
+            const int64_t r1 = std::min<int64_t>(r0 + rows, p->seqlen_q) - 1;
+            const int64_t lo = host_key_lo(p, r0 + dq), hi = host_key_hi(p, r1 + dq);
+            const int64_t n = hi >= lo ? hi / 32 - lo / 32 + 1 : 0;
+            if (k == 0) heaviest = std::max(heaviest, n);
+            total[k] += n;
+        }
+    }
+    const int64_t units = (int64_t)p->batch * p->heads_q;
+    const double whole = heaviest * tiles[0] == total[0]
+                             ? (double)((units * tiles[0] + cus - 1) / cus) * heaviest
+                             : std::max((double)heaviest, (double)units * total[0] / cus);
+    return whole > (dp <= 64 ? 1.2 : 1.3) * units * total[1] / (4.0 * cus);
+}
+
 KernelCfg single_cfg(int dp, bool bf16, int lds) {
     static const char* const names[2][4] = {
         {"mfa_fwd16x<f16,d32>", "mfa_fwd16x<f16,d64>", "mfa_fwd16x<f16,d96>", "mfa_fwd16x<f16,d128>"},
@@ -2581,8 +2779,9 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
     // Lq=26136 Lk=5 H=16: see the design notes)
     const bool tiny_keys = MFA_TK && p->tile_hint == MFA_TILE_AUTO && din != MFA_DTYPE_F32 && !paged &&
                            !single_call && split_keys == 0 && p->seqlen_k <= 32 && p->seqlen_q >= MFA_TK_MIN_ROWS;
+    const bool split32 = din == MFA_DTYPE_F32 && prefer_split32(p, dp, geom.cus);
     if (din == MFA_DTYPE_F32)
-        plan->cfg = bias ? select32<true>(dp, paged) : select32<false>(dp, paged);
+        plan->cfg = bias ? select32<true>(dp, split32, paged) : select32<false>(dp, split32, paged);
     else if (single_call)
         plan->cfg = single_cfg(dp, din == MFA_DTYPE_BF16, 0);  // (its LDS is plan_decode's choice)
     else if (tiny_keys && din == MFA_DTYPE_BF16)
@@ -2681,7 +2880,8 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
     const int R = p->heads_q / p->heads_kv;
     // The 4-wavefront 16-bit kernel packs 2 or 4 heads the same way (one or
     // two wavefronts per head), except for split-KV and paged calls.
-    const bool pack_pp = MFA_PP_HEAD_PACK && plan->cfg.threads == 8 * 64 && (R == 2 || R == 4 || R == 8);
+    const bool pack_pp = MFA_PP_HEAD_PACK && din != MFA_DTYPE_F32 && plan->cfg.threads == 8 * 64 &&
+                         (R == 2 || R == 4 || R == 8);
     const bool pack_4w = MFA_4W_HEAD_PACK && din != MFA_DTYPE_F32 && !tiny_keys && !paged &&
                          split_keys == 0 && plan->cfg.threads == kThreads && (R == 2 || R == 4);
     if (pack_pp || pack_4w) {
