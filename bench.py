@@ -347,7 +347,7 @@ def main():
     # steps faster than the GPU runs them, so the GPU runs the kernels back to
     # back and this is their average duration (plus the dispatch gap between
     # consecutive kernels).  A forward step is one launch; split-KV (config 8)
-    # adds the merge kernel and --backward runs three kernels, whose sum this
+    # adds the merge kernel and --backward runs two or three kernels, whose sum this
     # is.  (Events bracketing each call separately would add the event
     # records' own cost to every launch.)
     kernel_ms = ms_step
@@ -359,7 +359,7 @@ def main():
         # (the eight-wavefront dK/dV kernel above head dim 64; GQA adds the partial-sum kernel)
         dkdv = "mfa_bwd_dkdv8" if c["D"] > 64 else "mfa_bwd_dkdv"
         grouped = c["q"].shape[-2] != c["k"].shape[-2]
-        kname = f"mfa_bwd_dsum + {dkdv}" + (" + mfa_bwd_dkdv_sum" if grouped else "") + " + mfa_bwd_dq"
+        kname = f"mfa_bwd_dq + {dkdv}" + (" + mfa_bwd_dkdv_sum" if grouped else "")
     elif c["varlen"] is not None:
         cu, mx = c["varlen"]
         info = _kernel.launch_info_varlen(c["q"], c["k"], cu.shape[0] - 1, mx, mx, causal=c["kw"].get("causal", False))

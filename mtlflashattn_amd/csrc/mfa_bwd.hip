@@ -10,8 +10,7 @@
 //   dS = P * (dP - Dsum) * (1 - tanh^2)   (the last factor with soft-cap only),
 //   dQ = scale * dS K,  dK = scale * dS^T Q.
 //
-// Three kernels, no atomics (the result does not depend on scheduling):
-//  * mfa_bwd_dsum_kernel: Dsum per query row (fp32), 16 lanes per row.
+// Two kernels, no atomics (the result does not depend on scheduling), dQ first:
 //  * mfa_bwd_dkdv_kernel (head dims up to 64) / mfa_bwd_dkdv8_kernel (above):
 //    a workgroup owns 128 keys of one (sequence, K/V head), 32 per
 //    wavefront, with K and V resident in registers as MFMA B operands (four
@@ -24,7 +23,7 @@
 //    accumulators (rounded to 16 bits), with dO^T / Q^T read from LDS by
 //    ds_read_b64_tr_b16 -- the same operand scheme as the forward's O^T.
 //  * mfa_bwd_dq_kernel: a workgroup owns 128 query rows, 32 per wavefront,
-//    with Q and dO resident in registers; it walks the key blocks (64 keys,
+//    with Q and dO resident in registers; it forms their Dsum and walks the key blocks (64 keys,
 //    staged in LDS) its rows can see.  S^T = K Q^T and dP^T = V dO^T give
 //    lane = query, and dQ^T += K^T dS^T takes dS^T from the accumulators.
 // Tiles whose query-key pairs are all valid skip the masks; boundary tiles
@@ -242,38 +241,6 @@ __device__ __forceinline__ float transform(const KArgs& f, float x, float slope,
 }
 
 // ----------------------------------------------------------------------------
-// Dsum = rowsum(dO * O) in fp32: 16 lanes per row, 8 elements per lane.
-template <bool IS_BF16>
-__global__ void __launch_bounds__(kBThreads) mfa_bwd_dsum_kernel(BArgs a) {
-    const int bid = blockIdx.x;
-    const int unit = bid / a.T, tile = bid - unit * a.T;
-    const int b = unit / a.f.Hq, hq = unit - b * a.f.Hq;
-    const QView qv = q_view(a, b, hq);
-    const int row = tile * 16 + (threadIdx.x >> 4), sub = threadIdx.x & 15;
-    float acc = 0.f;
-    const int d0 = sub * 8;
-    if (row < qv.Lq && d0 < a.f.D) {
-        const u32x4_t o = *reinterpret_cast<const u32x4_t*>(qv.o + ((int64_t)row * a.f.os + d0) * 2);
-        const u32x4_t g = *reinterpret_cast<const u32x4_t*>(qv.dout + ((int64_t)row * a.dos + d0) * 2);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            acc = fmaf(Ops<IS_BF16>::to_f((uint16_t)(o[i] & 0xffff)), Ops<IS_BF16>::to_f((uint16_t)(g[i] & 0xffff)), acc);
-            acc = fmaf(Ops<IS_BF16>::to_f((uint16_t)(o[i] >> 16)), Ops<IS_BF16>::to_f((uint16_t)(g[i] >> 16)), acc);
-        }
-    }
-    acc += __shfl_xor(acc, 8);
-    acc += __shfl_xor(acc, 4);
-    acc += __shfl_xor(acc, 2);
-    acc += __shfl_xor(acc, 1);
-    if (sub == 0 && row < qv.Lq) {
-        if (a.dlse) {  // d lse / d s = P: enters as Dsum - dlse (same offset as the lse row)
-            const float* dl = a.dlse + (qv.lse - a.f.lse);
-            acc -= dl[row];
-        }
-        qv.dsum[row] = acc;
-    }
-}
-
 // Store rows of a transposed accumulator (lane = row `idx` of the output,
 // registers = columns d = 32*db + 8*g + 4*half + 0..3), scaled.
 template <int DB>
@@ -333,13 +300,16 @@ mfa_bwd_dkdv_kernel(BArgs a) {
 
     const KArgs& f = a.f;
     const int bid = blockIdx.x;
-    const int ktile = bid / (a.Ukv * a.G), rem = bid - ktile * (a.Ukv * a.G);
+    const int slot = bid / (a.Ukv * a.G), rem = bid - slot * (a.Ukv * a.G);
     const int unit = rem / a.G, grp = rem - unit * a.G;
     const int b = unit / f.Hkv, hkv = unit - b * f.Hkv;
     const KView kv = k_view(a, b, hkv);
     const int Lk = kv.Lk, D = f.D;
-    const int k0 = ktile * 128;
-    if (k0 >= Lk) return;
+    // the tiles with the most tiles after them first, over all sequences alike
+    // (under a causal mask, heaviest first): a sequence shorter than the longest
+    // skips the first slots, not the last
+    const int k0 = (slot - a.T + (Lk + 127) / 128) * 128;
+    if (k0 < 0 || k0 >= Lk) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, half = lane >> 5;
     const int key = k0 + wave * 32 + l32;  // this lane's key (B-operand / accumulator column)
@@ -614,13 +584,16 @@ __global__ void __launch_bounds__(kB8Threads) mfa_bwd_dkdv8_kernel(BArgs a) {
 
     const KArgs& f = a.f;
     const int bid = blockIdx.x;
-    const int ktile = bid / (a.Ukv * a.G), rem = bid - ktile * (a.Ukv * a.G);
+    const int slot = bid / (a.Ukv * a.G), rem = bid - slot * (a.Ukv * a.G);
     const int unit = rem / a.G, grp = rem - unit * a.G;
     const int b = unit / f.Hkv, hkv = unit - b * f.Hkv;
     const KView kv = k_view(a, b, hkv);
     const int Lk = kv.Lk, D = f.D;
-    const int k0 = ktile * 128;
-    if (k0 >= Lk) return;
+    // the tiles with the most tiles after them first, over all sequences alike
+    // (under a causal mask, heaviest first): a sequence shorter than the longest
+    // skips the first slots, not the last
+    const int k0 = (slot - a.T + (Lk + 127) / 128) * 128;
+    if (k0 < 0 || k0 >= Lk) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int kw = wave & 3, sb = wave >> 2;  // key block, query sub-block of each step
     const int l32 = lane & 31, half = lane >> 5;
@@ -983,21 +956,36 @@ mfa_bwd_dq_kernel(BArgs a) {
     const int q = wq0 + l32;             // this lane's query
     const bool qin = q < Lq;
 
-    // Q and dO rows as B operands (k-slots d = 16*s + 8*half + 0..7)
+    // Q and dO rows as B operands (k-slots d = 16*s + 8*half + 0..7), and the
+    // row's Dsum = rowsum(dO * O) - dlse in fp32: this kernel holds dO anyway,
+    // so it forms the row sums and stores them for the dK/dV kernel, which runs
+    // after it (a kernel of their own took 21.8 us for 12 sequences of 200 to
+    // 2048 rows, H=12 D=64, 14.1 us at L=8192 H=16 D=128, and a launch).
     op_t qf[DS], dof[DS];
+    float dsum = 0.f;
 #pragma unroll
     for (int s = 0; s < DS; ++s) {
         const int d = 16 * s + 8 * half;
-        u32x4_t qq = {0, 0, 0, 0}, gg = {0, 0, 0, 0};
+        u32x4_t qq = {0, 0, 0, 0}, gg = {0, 0, 0, 0}, oo = {0, 0, 0, 0};
         if (qin && d < D) {
             qq = *reinterpret_cast<const u32x4_t*>(qv.q + ((int64_t)q * f.qs + d) * 2);
             gg = *reinterpret_cast<const u32x4_t*>(qv.dout + ((int64_t)q * a.dos + d) * 2);
+            oo = *reinterpret_cast<const u32x4_t*>(qv.o + ((int64_t)q * f.os + d) * 2);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            dsum = fmaf(O::to_f((uint16_t)(oo[i] & 0xffff)), O::to_f((uint16_t)(gg[i] & 0xffff)), dsum);
+            dsum = fmaf(O::to_f((uint16_t)(oo[i] >> 16)), O::to_f((uint16_t)(gg[i] >> 16)), dsum);
         }
         qf[s] = __builtin_bit_cast(op_t, qq);
         dof[s] = __builtin_bit_cast(op_t, gg);
     }
     const float lse2 = qin ? lse2_of(qv.lse[q]) : INFINITY;
-    const float dsum = qin ? qv.dsum[q] : 0.f;
+    dsum = sum_halves(dsum);
+    if (qin) {
+        if (a.dlse) dsum -= a.dlse[(qv.lse - f.lse) + q];  // (same offset as the lse row)
+        if (half == 0) qv.dsum[q] = dsum;
+    }
     constexpr bool DFOLD = DP <= 64;  // registers allow the -Dsum vector
     f32x16_t negd;
 #pragma unroll
@@ -1190,7 +1178,7 @@ int bset_err(int code, const char* fmt, ...) {
 typedef void (*bkernel_fn)(BArgs);
 
 struct BwdKernels {
-    bkernel_fn dsum, dkdv, dq, dkdv_sum;
+    bkernel_fn dkdv, dq, dkdv_sum;
     int dkdv_threads;
     int dkdv_keys = 128;  // keys per dK/dV workgroup
     int dq_rows = 128;    // query rows per dQ workgroup
@@ -1199,7 +1187,6 @@ struct BwdKernels {
 template <int DP, bool IS_BF16>
 BwdKernels bwd_kernels(bool bias) {
     BwdKernels k;
-    k.dsum = mfa_bwd_dsum_kernel<IS_BF16>;
     k.dkdv_sum = mfa_bwd_dkdv_sum_kernel<IS_BF16>;
     if constexpr (DP > 64 && MFA_BWD_DKDV8) {
         k.dkdv = bias ? (bkernel_fn)mfa_bwd_dkdv8_kernel<DP, IS_BF16, true>
@@ -1226,7 +1213,6 @@ BwdKernels bwd_select(int dp, bool bias) {
 BwdKernels bwd32_select(int dp, bool bias) {
     const Bwd32Kernels f = mfa_bwd32_kernels(dp, bias);
     BwdKernels k;
-    k.dsum = reinterpret_cast<bkernel_fn>(f.dsum);
     k.dkdv = reinterpret_cast<bkernel_fn>(f.dkdv);
     k.dq = reinterpret_cast<bkernel_fn>(f.dq);
     k.dkdv_sum = nullptr;  // (one workgroup per K/V head's keys: no partials)
@@ -1241,7 +1227,7 @@ bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 struct BPlan {
     BArgs a;
     BwdKernels k;
-    int grid_dsum, grid_dkdv, grid_dq, grid_dkdv_sum;
+    int grid_dkdv, grid_dq, grid_dkdv_sum;
     int64_t dsum_bytes;  // workspace: row sums first, then the dK/dV partials
     int64_t ws_bytes;
     bool empty;
@@ -1380,13 +1366,11 @@ int make_bplan(const mfa_bwd_params* bp, BPlan* plan) {
     a.ws_ld = dp;
     const int64_t part_bytes = a.G > 1 ? 2 * a.G * part : 0;
     plan->ws_bytes = plan->empty ? 0 : plan->dsum_bytes + part_bytes;
-    const int64_t g1 = (int64_t)f.U * ((p->seqlen_q + 15) / 16);
     const int kt = plan->k.dkdv_keys, qt = plan->k.dq_rows;
     const int64_t g2 = (int64_t)a.Ukv * a.G * ((p->seqlen_k + kt - 1) / kt);
     const int64_t g3 = (int64_t)f.U * ((p->seqlen_q + qt - 1) / qt);
-    if (g1 > 0x7fffffffLL || g2 > 0x7fffffffLL || g3 > 0x7fffffffLL)
+    if (g2 > 0x7fffffffLL || g3 > 0x7fffffffLL)
         return bset_err(MFA_ERR_INVALID, "mfa_bwd: problem too large");
-    plan->grid_dsum = (int)g1;
     plan->grid_dkdv = (int)g2;
     plan->grid_dq = (int)g3;
     const int64_t g4 = ((int64_t)a.Ukv * p->seqlen_k * (D / 4) + kBThreads - 1) / kBThreads;
@@ -1438,15 +1422,14 @@ int mfa_bwd(const mfa_bwd_params* params, void* workspace, int64_t workspace_byt
     const int cus = params->fwd.dtype_in == MFA_DTYPE_F32 && params->fwd.causal && a.ws_ld <= kB32PairDim
                         ? mfa_chip_cus(stream) : 0;
     auto fold = [&](int grid, int units) { return grid > cus && grid <= 2 * cus ? std::max(1, cus / units) : 0; };
-    a.T = (params->fwd.seqlen_q + 15) / 16;
-    hipLaunchKernelGGL(plan.k.dsum, dim3(plan.grid_dsum), dim3(kBThreads), 0, st, a);
+    // dQ first: it stores the row sums that dK/dV read
+    a.T = (params->fwd.seqlen_q + plan.k.dq_rows - 1) / plan.k.dq_rows;
+    a.fold = fold(plan.grid_dq, a.f.U);
+    hipLaunchKernelGGL(plan.k.dq, dim3(plan.grid_dq), dim3(kBThreads), 0, st, a);
     a.T = (params->fwd.seqlen_k + plan.k.dkdv_keys - 1) / plan.k.dkdv_keys;
     a.fold = fold(plan.grid_dkdv, a.Ukv * a.G);
     hipLaunchKernelGGL(plan.k.dkdv, dim3(plan.grid_dkdv), dim3(plan.k.dkdv_threads), 0, st, a);
     if (a.G > 1) hipLaunchKernelGGL(plan.k.dkdv_sum, dim3(plan.grid_dkdv_sum), dim3(kBThreads), 0, st, a);
-    a.T = (params->fwd.seqlen_q + plan.k.dq_rows - 1) / plan.k.dq_rows;
-    a.fold = fold(plan.grid_dq, a.f.U);
-    hipLaunchKernelGGL(plan.k.dq, dim3(plan.grid_dq), dim3(kBThreads), 0, st, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return bset_err(MFA_ERR_LAUNCH, "mfa_bwd: launch failed: %s", hipGetErrorString(e));
     return MFA_OK;

@@ -2,10 +2,10 @@
 // fp32 q, k, v, o and dO in, fp32 dq, dk and dv out, every product and sum in
 // fp32 (v_mfma_f32_32x32x2_f32), the fp32 forward's score transform.
 //
-// The decomposition is that of the 16-bit kernels (mfa_bwd.hip): Dsum; dK/dV
-// for a block of keys of one (sequence, K/V head), walking every query block
-// of its head group that sees them; dQ for a block of query rows, walking the
-// key blocks they see.  No atomics: a fixed order of sums.
+// The decomposition is that of the 16-bit kernels (mfa_bwd.hip): dQ (and Dsum)
+// for a block of query rows, walking the key blocks they see; then dK/dV for a
+// block of keys of one (sequence, K/V head), walking every query block of its
+// head group that sees them.  No atomics: a fixed order of sums.
 //
 // What bounds them: the matrix pipe.  One 32 x 32 tile of (query, key) pairs
 // is 2 DP MFMAs of 64 cycles in dK/dV (1.5 DP in dQ), against ~300 vector
@@ -115,39 +115,6 @@ __device__ __forceinline__ void pair32(const KArgs& f, float lse2, float dsum, f
     ds = p * (dp - dsum) * dx;
 }
 
-// Dsum = rowsum(dO * O) - dlse in fp32: 16 lanes per row, 8 elements per lane.
-__global__ void __launch_bounds__(kBThreads) mfa_bwd32_dsum_kernel(BArgs a) {
-    const int bid = blockIdx.x;
-    const int unit = bid / a.T, tile = bid - unit * a.T;
-    const int b = unit / a.f.Hq, hq = unit - b * a.f.Hq;
-    const QView32 qv = q_view32(a, b, hq);
-    const int row = tile * 16 + (threadIdx.x >> 4), sub = threadIdx.x & 15;
-    float acc = 0.f;
-    const int d0 = sub * 8;
-    if (row < qv.Lq && d0 < a.f.D) {  // (D is a multiple of 8)
-#pragma unroll
-        for (int e = 0; e < 8; e += 4) {
-            const float4 o = *reinterpret_cast<const float4*>(qv.o + (int64_t)row * a.f.os + d0 + e);
-            const float4 g = *reinterpret_cast<const float4*>(qv.dout + (int64_t)row * a.dos + d0 + e);
-            acc = fmaf(o.x, g.x, acc);
-            acc = fmaf(o.y, g.y, acc);
-            acc = fmaf(o.z, g.z, acc);
-            acc = fmaf(o.w, g.w, acc);
-        }
-    }
-    acc += __shfl_xor(acc, 8);
-    acc += __shfl_xor(acc, 4);
-    acc += __shfl_xor(acc, 2);
-    acc += __shfl_xor(acc, 1);
-    if (sub == 0 && row < qv.Lq) {
-        if (a.dlse) {
-            const float* dl = a.dlse + (qv.lse - a.f.lse);
-            acc -= dl[row];
-        }
-        qv.dsum[row] = acc;
-    }
-}
-
 // dQ of 32 query rows (lane = row): dQ^T = sum over key blocks of K^T dS'^T
 // (dS' = dS * d score / d(q.k)).  Per block: dP^T = V dO^T, S^T = K Q^T, dS',
 // dQ^T; V's tile is free after the first product and K's after the last, so
@@ -200,7 +167,24 @@ mfa_bwd32_dq_kernel(BArgs a) {
     row_operand<DP>(qf, qv.q + (int64_t)row * f.qs, in, D, half);
     row_operand<DP>(gf, qv.dout + (int64_t)row * a.dos, in, D, half);
     const float lse2 = in ? lse2_of(qv.lse[row]) : INFINITY;
-    const float dsum = in ? qv.dsum[row] : 0.f;
+    // the row's Dsum = rowsum(dO * O) - dlse, also stored for the dK/dV kernel,
+    // which runs after this one
+    float dsum = 0.f;
+#pragma unroll
+    for (int s = 0; s < DP / 2; s += 4) {
+        const int d = s + half * (DP / 2);
+        float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (in && d < D) w = *reinterpret_cast<const float4*>(qv.o + (int64_t)row * f.os + d);
+        dsum = fmaf(w.x, gf[s], dsum);
+        dsum = fmaf(w.y, gf[s + 1], dsum);
+        dsum = fmaf(w.z, gf[s + 2], dsum);
+        dsum = fmaf(w.w, gf[s + 3], dsum);
+    }
+    dsum = sum_halves(dsum);
+    if (in) {
+        if (a.dlse) dsum -= a.dlse[(qv.lse - f.lse) + row];  // (same offset as the lse row)
+        if (half == 0 && tid < 64) qv.dsum[row] = dsum;
+    }
     const int center = row + dq, lo = key_lo(f, center), hi = in ? key_hi(f, center, Lk) : -1;
     const int lo_last = key_lo(f, q0 + nrow - 1 + dq), hi_first = key_hi(f, q0 + dq, Lk);
     const float slope = BIAS && f.alibi ? f.alibi[b * f.alibi_bstride + hq] : 0.f;
@@ -266,12 +250,13 @@ mfa_bwd32_dkdv_kernel(BArgs a) {
     const KArgs& f = a.f;
     // the first (under a causal mask the heaviest) keys of every unit first
     const int slot = blockIdx.x / a.Ukv, ukv = blockIdx.x - slot * a.Ukv;
-    const int ktile = fold_slot(a, slot);
     const int b = ukv / f.Hkv, hkv = ukv - b * f.Hkv;
     const KView32 kv = k_view32(a, b, hkv);
     const int Lk = kv.Lk, D = f.D;
-    const int k0 = ktile * kB32Keys;
-    if (k0 >= Lk) return;
+    // (a sequence shorter than the longest skips the first slots: the heaviest
+    // tiles of all sequences run first)
+    const int k0 = (fold_slot(a, slot) - a.T + (Lk + kB32Keys - 1) / kB32Keys) * kB32Keys;
+    if (k0 < 0 || k0 >= Lk) return;
     const int nk = min(kB32Keys, Lk - k0), k1 = k0 + nk - 1;
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -393,7 +378,6 @@ template <int DP>
 Bwd32Kernels kernels32(bool bias) {
     typedef void (*fn)(BArgs);
     return Bwd32Kernels{
-        (void*)mfa_bwd32_dsum_kernel,
         (void*)(bias ? (fn)mfa_bwd32_dkdv_kernel<DP, true> : (fn)mfa_bwd32_dkdv_kernel<DP, false>),
         (void*)(bias ? (fn)mfa_bwd32_dq_kernel<DP, true> : (fn)mfa_bwd32_dq_kernel<DP, false>)};
 }

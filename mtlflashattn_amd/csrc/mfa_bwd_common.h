@@ -9,7 +9,7 @@
 constexpr int kB32Rows = 32;  // query rows per dQ workgroup
 constexpr int kB32Keys = 32;  // keys per dK/dV workgroup
 struct Bwd32Kernels {
-    void *dsum, *dkdv, *dq;
+    void *dkdv, *dq;
 };
 // Two workgroups of these kernels share a CU up to this padded head dim, one above.
 constexpr int kB32PairDim = 64;
@@ -33,7 +33,7 @@ struct BArgs {
     float* dsum;       // [B*Hq][Lq] rowsum(dO * O) - dlse
     const float* dlse; // gradient of lse (softmax_lse layout), or NULL
     int32_t grad_f32;  // dq/dk/dv written as fp32
-    int32_t T;         // tiles per unit (dsum: 16-row groups; dK/dV: key tiles; dQ: query tiles)
+    int32_t T;         // tiles per unit (dK/dV: key tiles; dQ: query tiles)
     int32_t fold;      // fp32 kernels: tile slots from here on run in reverse order (0: off)
     int32_t Ukv;       // (sequence, K/V head) units = B * Hkv
     // grouped-query heads split over dK/dV workgroups: G groups of R/G query
