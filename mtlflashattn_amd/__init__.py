@@ -99,8 +99,15 @@ def flash_attn_func(
     q: [B, Lq, Hq, D]; k, v: [B, Lk, Hkv, D] (heads-third, CUDA flash-attn layout).
     Hkv must divide Hq (GQA/MQA). Returns [B, Lq, Hq, D] in q.dtype.
     """
+    return _attn_func(None, q, k, v, dropout_p, softmax_scale, causal, window_size, softcap, alibi_slopes,
+                      deterministic, return_attn_probs)
+
+
+def _attn_func(packed, q, k, v, dropout_p=0.0, softmax_scale=None, causal=False, window_size=(-1, -1), softcap=0.0,
+               alibi_slopes=None, deterministic=False, return_attn_probs=False):
+    """flash_attn_func; packed: the tensors q, k, v are views of, (qkv,) or (q, kv), or None."""
     _check_supported(q, k, v, dropout_p, window_size, softcap, alibi_slopes, deterministic, return_attn_probs)
-    return _dense(q, k, v, softmax_scale, causal, window_size, softcap, alibi_slopes, False)
+    return _dense(q, k, v, softmax_scale, causal, window_size, softcap, alibi_slopes, False, packed)
 
 
 def flash_attn_func_with_lse(q, k, v, softmax_scale=None, causal=False, window_size=(-1, -1), softcap=0.0,
@@ -118,7 +125,7 @@ def flash_attn_func_with_lse(q, k, v, softmax_scale=None, causal=False, window_s
     return _dense(q, k, v, softmax_scale, causal, window_size, softcap, alibi_slopes, True)
 
 
-def _dense(q, k, v, softmax_scale, causal, window_size, softcap, alibi_slopes, return_lse):
+def _dense(q, k, v, softmax_scale, causal, window_size, softcap, alibi_slopes, return_lse, packed=None):
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
         raise ValueError(f"mtlflashattn_amd: expected 4-D [B,S,H,D] tensors, got q.dim()={q.dim()}")
     _kernel._check_qkv_shapes(q, k, v, h_axis=2, s_axis=1)
@@ -126,6 +133,7 @@ def _dense(q, k, v, softmax_scale, causal, window_size, softcap, alibi_slopes, r
     return forward_bshd(
         q, k, v, scale=scale, causal=causal, softcap=softcap,
         window_left=window_size[0], window_right=window_size[1], alibi_slopes=alibi_slopes, return_lse=return_lse,
+        packed=packed,
     )
 
 
@@ -164,9 +172,18 @@ def flash_attn_varlen_func(
     the rows that see them are wrong; MTLFLASHATTN_CHECK_PAGES=1 checks the
     ids on the host and raises ValueError instead.
     """
+    return _attn_varlen_func(None, q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p,
+                             softmax_scale, causal, window_size, softcap, alibi_slopes, deterministic,
+                             return_attn_probs, block_table)
+
+
+def _attn_varlen_func(packed, q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p=0.0,
+                      softmax_scale=None, causal=False, window_size=(-1, -1), softcap=0.0, alibi_slopes=None,
+                      deterministic=False, return_attn_probs=False, block_table=None):
+    """flash_attn_varlen_func; packed: as in _attn_func."""
     _check_supported(q, k, v, dropout_p, window_size, softcap, alibi_slopes, deterministic, return_attn_probs)
     return _varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, softmax_scale, causal, window_size, softcap, alibi_slopes,
-                   block_table, False)
+                   block_table, False, packed)
 
 
 def flash_attn_varlen_func_with_lse(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
@@ -183,7 +200,7 @@ def flash_attn_varlen_func_with_lse(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seq
 
 
 def _varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, softmax_scale, causal, window_size, softcap, alibi_slopes,
-            block_table, return_lse):
+            block_table, return_lse, packed=None):
     paged = block_table is not None
     if q.dim() != 3 or k.dim() != (4 if paged else 3) or v.dim() != (4 if paged else 3):
         if paged:
@@ -231,7 +248,7 @@ def _varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, softmax_scale, causal, window_s
         q, k, v, cu_seqlens_q, cu_seqlens_k, max(lens_q, default=0), max(lens_k, default=0),
         scale=scale, causal=causal, softcap=softcap, window_left=window_size[0],
         window_right=window_size[1], alibi_slopes=alibi_slopes, return_lse=return_lse, block_table=block_table,
-        no_single_rows=1 not in lens_q,
+        no_single_rows=1 not in lens_q, packed=packed,
     )
 
 
@@ -319,7 +336,7 @@ def flash_attn_qkvpacked_func(qkv, *args, **kwargs):
     if qkv.dim() != 5 or qkv.shape[2] != 3:
         raise ValueError(f"mtlflashattn_amd: expected qkv [B,S,3,H,D], got {tuple(qkv.shape)}")
     q, k, v = qkv.unbind(dim=2)
-    return flash_attn_func(q, k, v, *args, **kwargs)
+    return _attn_func((qkv,), q, k, v, *args, **kwargs)
 
 
 def flash_attn_kvpacked_func(q, kv, *args, **kwargs):
@@ -327,7 +344,7 @@ def flash_attn_kvpacked_func(q, kv, *args, **kwargs):
     if kv.dim() != 5 or kv.shape[2] != 2:
         raise ValueError(f"mtlflashattn_amd: expected kv [B,S,2,H,D], got {tuple(kv.shape)}")
     k, v = kv.unbind(dim=2)
-    return flash_attn_func(q, k, v, *args, **kwargs)
+    return _attn_func((q, kv), q, k, v, *args, **kwargs)
 
 
 def flash_attn_varlen_qkvpacked_func(qkv, cu_seqlens, max_seqlen, *args, **kwargs):
@@ -335,7 +352,7 @@ def flash_attn_varlen_qkvpacked_func(qkv, cu_seqlens, max_seqlen, *args, **kwarg
     if qkv.dim() != 4 or qkv.shape[1] != 3:
         raise ValueError(f"mtlflashattn_amd: expected qkv [total,3,H,D], got {tuple(qkv.shape)}")
     q, k, v = qkv.unbind(dim=1)
-    return flash_attn_varlen_func(q, k, v, cu_seqlens, cu_seqlens, max_seqlen, max_seqlen, *args, **kwargs)
+    return _attn_varlen_func((qkv,), q, k, v, cu_seqlens, cu_seqlens, max_seqlen, max_seqlen, *args, **kwargs)
 
 
 def flash_attn_varlen_kvpacked_func(q, kv, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, *args, **kwargs):
@@ -343,4 +360,5 @@ def flash_attn_varlen_kvpacked_func(q, kv, cu_seqlens_q, cu_seqlens_k, max_seqle
     if kv.dim() != 4 or kv.shape[1] != 2:
         raise ValueError(f"mtlflashattn_amd: expected kv [total,2,H,D], got {tuple(kv.shape)}")
     k, v = kv.unbind(dim=1)
-    return flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, *args, **kwargs)
+    return _attn_varlen_func((q, kv), q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, *args,
+                             **kwargs)

@@ -423,8 +423,8 @@ def flash_attn_forward(q, k, v, scale, causal, softcap=0.0, window_left=-1, wind
         raise NotImplementedError(f"mtlflashattn_amd: head_dim {D} > {MAX_HEAD_DIM}")
     if _needs_grad(q, k, v) and _out_dtype(q, out_dtype) == q.dtype:
         # differentiable path (heads-third views of the same tensors)
-        o, lse = _FlashAttnFn.apply(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), scale, causal,
-                                    softcap, window_left, window_right, alibi_slopes)
+        o, lse = _FlashAttnFn.apply(scale, causal, softcap, window_left, window_right, alibi_slopes,
+                                    q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2))
         o = o.transpose(1, 2).contiguous()
         return (o, lse) if return_lse else o
     out = torch.empty(B, Hq, Lq, D, dtype=_out_dtype(q, out_dtype), device=q.device)
@@ -436,13 +436,14 @@ def flash_attn_forward(q, k, v, scale, causal, softcap=0.0, window_left=-1, wind
 
 
 def forward_bshd(q, k, v, scale, causal, softcap=0.0, window_left=-1, window_right=-1,
-                 alibi_slopes=None, out_dtype=None, return_lse=False):
+                 alibi_slopes=None, out_dtype=None, return_lse=False, packed=None):
     """Heads-third forward: q [B,Lq,Hq,D], k/v [B,Lk,Hkv,D] -> [B,Lq,Hq,D].
 
     Same result as flash_attn_forward on the transposed views followed by
     `.transpose(1, 2).contiguous()` (metal_flash_attn/__init__.py:93-99), but
     the kernel writes the heads-third output directly (no layout copies).
-    return_lse=True returns (out, lse [B,Hq,Lq] fp32).
+    return_lse=True returns (out, lse [B,Hq,Lq] fp32).  packed: the tensors
+    q, k, v are views of, (q, kv) or (qkv,), as _split_packed takes them.
     """
     if _trace_enabled():
         _record_trace(q.dtype, q.shape[-1], q.shape[1], k.shape[1], causal)
@@ -452,7 +453,8 @@ def forward_bshd(q, k, v, scale, causal, softcap=0.0, window_left=-1, window_rig
     B, Lq, Hq, D = q.shape
     if _needs_grad(q, k, v) and _out_dtype(q, out_dtype) == q.dtype:
         _alibi_arg(alibi_slopes, B, Hq, q.device)  # validate before autograd records anything
-        o, lse = _FlashAttnFn.apply(q, k, v, scale, causal, softcap, window_left, window_right, alibi_slopes)
+        o, lse = _FlashAttnFn.apply(scale, causal, softcap, window_left, window_right, alibi_slopes,
+                                    *(packed or (q, k, v)))
         return (o, lse) if return_lse else o
     alibi, bstride = _alibi_arg(alibi_slopes, B, Hq, q.device)
     out = torch.empty(B, Lq, Hq, D, dtype=_out_dtype(q, out_dtype), device=q.device)
@@ -464,7 +466,7 @@ def forward_bshd(q, k, v, scale, causal, softcap=0.0, window_left=-1, window_rig
 
 def forward_varlen(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap=0.0, window_left=-1,
                    window_right=-1, alibi_slopes=None, out_dtype=None, return_lse=False, block_table=None,
-                   _grad=True, no_single_rows=False):
+                   _grad=True, no_single_rows=False, packed=None):
     """Packed varlen forward in ONE launch: q [Tq,Hq,D], k/v [Tk,Hkv,D].
 
     cu_q/cu_k: int32 [batch+1] device tensors; max_q/max_k: the longest
@@ -477,7 +479,7 @@ def forward_varlen(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap=0.0
     table, q.dtype output) go through the HIP backward.  no_single_rows: the
     caller knows no sequence has exactly one query row (the library then
     skips the single-row launch for such sequences; a one-row sequence would
-    be left unwritten).
+    be left unwritten).  packed: as in forward_bshd.
     """
     batch = cu_q.shape[0] - 1
     Hq = q.shape[1]
@@ -493,8 +495,8 @@ def forward_varlen(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap=0.0
         raise NotImplementedError("mtlflashattn_amd: paged K/V (block_table) calls are forward-only; "
                                   "run them under torch.no_grad() or without inputs that require grad")
     if _grad and block_table is None and _needs_grad(q, k, v) and _out_dtype(q, out_dtype) == q.dtype:
-        o, lse = _FlashAttnVarlenFn.apply(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap, window_left,
-                                          window_right, alibi_slopes, no_single_rows)
+        o, lse = _FlashAttnVarlenFn.apply(cu_q, cu_k, max_q, max_k, scale, causal, softcap, window_left,
+                                          window_right, alibi_slopes, no_single_rows, *(packed or (q, k, v)))
         return (o, lse) if return_lse else o
     out = torch.empty(q.shape, dtype=_out_dtype(q, out_dtype), device=q.device)
     lse = torch.empty(Hq, q.shape[0], dtype=torch.float32, device=q.device) if return_lse else None
@@ -521,13 +523,14 @@ def _needs_grad(*tensors):
 
 
 def _run_bwd(q, k, v, out, dout, lse, *, scale, causal, softcap, window_left, window_right, alibi, alibi_bstride,
-             cu_q=None, cu_k=None, seqlen_q=None, seqlen_k=None, grad_f32=False, dlse=None):
+             cu_q=None, cu_k=None, seqlen_q=None, seqlen_k=None, grad_f32=False, dlse=None, into=None):
     """(dq, dk, dv) of the forward on [B, S, H, D] views (varlen: [1, T, H, D]).
 
     out: the forward's output in q.dtype; lse: its softmax_lse ([B, Hq, Lq]
     dense, [Hq, T] varlen); dlse: optional gradient of lse (same shape).
     Returns new tensors shaped like q, k, v in q.dtype (grad_f32=True: fp32,
-    the parity mode).
+    the parity mode).  into: (dq, dk, dv) to write and return instead, views
+    with a contiguous head dim of freshly allocated tensors (None: allocate).
     """
     _kernel_mode()
     _check_device(q, k, v, out, dout)
@@ -538,16 +541,18 @@ def _run_bwd(q, k, v, out, dout, lse, *, scale, causal, softcap, window_left, wi
     Lq = int(seqlen_q) if varlen else Sq
     Lk = int(seqlen_k) if varlen else k.shape[1]
     gdt = torch.float32 if grad_f32 else q.dtype
+    into = into or (None, None, None)
     if batch == 0 or Lq == 0 or Lk == 0 or Hq == 0 or q.numel() == 0 or k.numel() == 0:
-        return tuple(torch.zeros(t.shape, dtype=gdt, device=t.device) for t in (q, k, v))
+        return tuple(torch.zeros(t.shape, dtype=gdt, device=t.device) if g is None else g.zero_()
+                     for t, g in zip((q, k, v), into))
     Dp = -(-D // 8) * 8
     ts = [q, k, v, out, dout.to(q.dtype)]
     if Dp != D:
         ts = [F.pad(t, (0, Dp - D)) for t in ts]
     q_, k_, v_, o_, do_ = (_abi_operand(t) for t in ts)
-    dq = torch.empty(q_.shape, dtype=gdt, device=q.device)
-    dk = torch.empty(k_.shape, dtype=gdt, device=q.device)
-    dv = torch.empty(v_.shape, dtype=gdt, device=q.device)
+    # (a padded head dim, or a view the library cannot address: through a tensor of its own)
+    dq, dk, dv = (torch.empty(t.shape, dtype=gdt, device=q.device) if g is None or Dp != D or not _fits_abi(g) else g
+                  for t, g in zip((q_, k_, v_), into))
 
     bp = _hip.MfaBwdParams()
     p = bp.fwd
@@ -589,22 +594,44 @@ def _run_bwd(q, k, v, out, dout, lse, *, scale, causal, softcap, window_left, wi
         _hip.bwd(bp, ws.data_ptr(), nbytes, torch._C._cuda_getCurrentRawStream(device.index))
     if Dp != D:
         dq, dk, dv = dq[..., :D], dk[..., :D], dv[..., :D]
-    return dq, dk, dv
+    return tuple(t if g is None or g is t else g.copy_(t) for t, g in zip((dq, dk, dv), into))
+
+
+# Inputs of the autograd functions as the caller holds them: (q, k, v), (q, kv)
+# with kv [..., 2, H, D], or (qkv,) with qkv [..., 3, H, D].  The functions take
+# the packed tensors themselves, so their gradients are written in place in one
+# packed tensor each; views split off before would have autograd stack dq, dk
+# and dv (a pass over all three: 40 us for 13600 tokens x 12 heads x 64).
+def _split_packed(ts):
+    """(q, k, v) views of packed or separate inputs."""
+    if len(ts) == 3:
+        return tuple(ts)
+    if len(ts) == 2:
+        return (ts[0], *ts[1].unbind(-3))
+    return ts[0].unbind(-3)
+
+
+def _packed_grads(ts):
+    """New gradient tensors for packed inputs, None for separate ones (whose
+    gradients the backward allocates itself)."""
+    return tuple(torch.empty(t.shape, dtype=t.dtype, device=t.device) for t in ts) if len(ts) < 3 else None
 
 
 class _FlashAttnFn(torch.autograd.Function):
     """Heads-third dense attention with the HIP backward; returns (out, lse),
-    both differentiable (a gradient on lse enters the backward's row sums)."""
+    both differentiable (a gradient on lse enters the backward's row sums).
+    The last inputs are the tensors: q, k, v, or packed (_split_packed)."""
 
     @staticmethod
-    def forward(ctx, q, k, v, scale, causal, softcap, window_left, window_right, alibi_slopes):
+    def forward(ctx, scale, causal, softcap, window_left, window_right, alibi_slopes, *ts):
+        q, k, v = _split_packed(ts)
         B, Lq, Hq, D = q.shape
         alibi, bstride = _alibi_arg(alibi_slopes, B, Hq, q.device)
         out = torch.empty(B, Lq, Hq, D, dtype=q.dtype, device=q.device)
         lse = torch.empty(B, Hq, Lq, dtype=torch.float32, device=q.device)
         _run(q, k, v, out, scale=scale, causal=causal, softcap=softcap, window_left=window_left,
              window_right=window_right, alibi=alibi, alibi_bstride=bstride, lse=lse)
-        ctx.save_for_backward(q, k, v, out, lse)
+        ctx.save_for_backward(out, lse, *ts)
         ctx.cfg = dict(scale=scale, causal=causal, softcap=softcap, window_left=window_left,
                        window_right=window_right, alibi=alibi, alibi_bstride=bstride)
         ctx.set_materialize_grads(False)
@@ -612,20 +639,22 @@ class _FlashAttnFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout, dlse):
-        q, k, v, out, lse = ctx.saved_tensors
+        out, lse, *ts = ctx.saved_tensors
         if dout is None:
             dout = torch.zeros_like(out)
-        dq, dk, dv = _run_bwd(q, k, v, out, dout, lse, dlse=dlse, **ctx.cfg)
-        return dq, dk, dv, None, None, None, None, None, None
+        grads = _packed_grads(ts)
+        dqkv = _run_bwd(*_split_packed(ts), out, dout, lse, dlse=dlse, into=grads and _split_packed(grads), **ctx.cfg)
+        return None, None, None, None, None, None, *(grads or dqkv)
 
 
 class _FlashAttnVarlenFn(torch.autograd.Function):
     """Packed varlen attention with the HIP backward; returns (out, lse [Hq, T]),
-    both differentiable."""
+    both differentiable.  The last inputs are the tensors, as in _FlashAttnFn."""
 
     @staticmethod
-    def forward(ctx, q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap, window_left, window_right,
-                alibi_slopes, no_single_rows=False):
+    def forward(ctx, cu_q, cu_k, max_q, max_k, scale, causal, softcap, window_left, window_right, alibi_slopes,
+                no_single_rows, *ts):
+        q, k, v = _split_packed(ts)
         out, lse = forward_varlen(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap, window_left,
                                   window_right, alibi_slopes, return_lse=True, _grad=False,
                                   no_single_rows=no_single_rows)
@@ -633,7 +662,7 @@ class _FlashAttnVarlenFn(torch.autograd.Function):
         alibi, bstride = _alibi_arg(alibi_slopes, batch, Hq, q.device)
         cu_q = cu_q.to(device=q.device, dtype=torch.int32).contiguous()
         cu_k = cu_k.to(device=q.device, dtype=torch.int32).contiguous()
-        ctx.save_for_backward(q, k, v, out, lse, cu_q, cu_k)
+        ctx.save_for_backward(out, lse, cu_q, cu_k, *ts)
         ctx.cfg = dict(scale=scale, causal=causal, softcap=softcap, window_left=window_left,
                        window_right=window_right, alibi=alibi, alibi_bstride=bstride, seqlen_q=max_q,
                        seqlen_k=max_k)
@@ -642,12 +671,14 @@ class _FlashAttnVarlenFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout, dlse):
-        q, k, v, out, lse, cu_q, cu_k = ctx.saved_tensors
+        out, lse, cu_q, cu_k, *ts = ctx.saved_tensors
         if dout is None:
             dout = torch.zeros_like(out)
-        dq, dk, dv = _run_bwd(q[None], k[None], v[None], out[None], dout[None], lse, cu_q=cu_q, cu_k=cu_k,
-                              dlse=dlse, **ctx.cfg)
-        return dq[0], dk[0], dv[0], None, None, None, None, None, None, None, None, None, None, None
+        grads = _packed_grads(ts)
+        q, k, v = _split_packed(ts)
+        dqkv = _run_bwd(q[None], k[None], v[None], out[None], dout[None], lse, cu_q=cu_q, cu_k=cu_k, dlse=dlse,
+                        into=grads and tuple(g[None] for g in _split_packed(grads)), **ctx.cfg)
+        return (None,) * 11 + (grads or tuple(g[0] for g in dqkv))
 
 
 def _plain(*tensors) -> bool:
