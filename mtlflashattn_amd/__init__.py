@@ -133,7 +133,7 @@ def _dense(q, k, v, softmax_scale, causal, window_size, softcap, alibi_slopes, r
     return forward_bshd(
         q, k, v, scale=scale, causal=causal, softcap=softcap,
         window_left=window_size[0], window_right=window_size[1], alibi_slopes=alibi_slopes, return_lse=return_lse,
-        packed=packed,
+        packed=packed, checked=True,
     )
 
 
@@ -275,7 +275,10 @@ def _host_prefix_sums(cu_seqlens_q, cu_seqlens_k):
             and cached[2] == versions):
         return cached[3], cached[4]
     n = cu_seqlens_q.shape[0]
-    cu = torch.cat([cu_seqlens_q.reshape(-1).to(torch.int64), cu_seqlens_k.reshape(-1).to(torch.int64)]).tolist()
+    ts = [cu_seqlens_q.reshape(-1), cu_seqlens_k.reshape(-1)]
+    if not (ts[0].dtype is torch.int32 and ts[1].dtype is torch.int32):
+        ts = [t.to(torch.int64) for t in ts]
+    cu = torch.cat(ts).tolist()
     cu_q, cu_k = cu[:n], cu[n:]
     if versions is not None:
         _cu_host = (cu_seqlens_q, cu_seqlens_k, versions, cu_q, cu_k)

@@ -46,7 +46,10 @@ _c_ptr = ctypes.c_void_p
 
 
 class MfaFwdParams(ctypes.Structure):
-    """Mirror of `mfa_fwd_params` (include/mfa.h)."""
+    """Mirror of `mfa_fwd_params` (include/mfa.h).  workspace: bytes of its
+    split-KV workspace where the caller knows them (not part of the struct)."""
+
+    workspace = None
 
     _fields_ = [
         ("q", _c_ptr), ("k", _c_ptr), ("v", _c_ptr), ("o", _c_ptr),

@@ -61,7 +61,10 @@ _SPLIT_KEYS = None
 
 
 def _kernel_mode() -> str:
-    mode = os.environ.get("MTLFLASHATTN_KERNEL", "auto").lower()
+    mode = os.environ.get("MTLFLASHATTN_KERNEL")
+    if mode is None:
+        return "hip"
+    mode = mode.lower()
     if mode not in ("auto", "hip") and mode not in _warned_modes:
         _warned_modes.add(mode)
         what = "a Metal tier" if mode in _KNOWN_MODES else "unknown"
@@ -81,7 +84,8 @@ _trace = {}
 
 
 def _trace_enabled() -> bool:
-    return os.environ.get("MTLFLASHATTN_TRACE", "").lower() in ("1", "on", "true", "yes")
+    v = os.environ.get("MTLFLASHATTN_TRACE")
+    return v is not None and v.lower() in ("1", "on", "true", "yes")
 
 
 def _effective_kernel_label(q, k, v) -> str:
@@ -145,16 +149,17 @@ def _check_qkv_shapes(q, k, v, h_axis, s_axis):
     and a K/V head count that divides the query head count (CUDA flash-attn
     and stock SDPA reject the rest; the kernel takes B from q and the K/V
     head count from k, so a mismatch must never reach it)."""
-    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
+    qs, ks, vs = q.shape, k.shape, v.shape
+    if len(qs) != 4 or len(ks) != 4 or len(vs) != 4:
         raise ValueError(f"mtlflashattn_amd: expected 4-D q/k/v, got {q.dim()}/{k.dim()}/{v.dim()} dims")
-    if not (q.shape[0] == k.shape[0] == v.shape[0]):
-        raise ValueError(f"mtlflashattn_amd: batch mismatch (q {q.shape[0]}, k {k.shape[0]}, v {v.shape[0]})")
-    Hq, Hkv = q.shape[h_axis], k.shape[h_axis]
+    if not (qs[0] == ks[0] == vs[0]):
+        raise ValueError(f"mtlflashattn_amd: batch mismatch (q {qs[0]}, k {ks[0]}, v {vs[0]})")
+    Hq, Hkv = qs[h_axis], ks[h_axis]
     if Hkv == 0 or Hq % Hkv != 0:
         raise ValueError(f"mtlflashattn_amd: num_heads_kv ({Hkv}) must divide num_heads_q ({Hq})")
-    if v.shape[h_axis] != Hkv:
-        raise ValueError(f"mtlflashattn_amd: k has {Hkv} heads, v {v.shape[h_axis]}")
-    if k.shape[s_axis] != v.shape[s_axis]:
+    if vs[h_axis] != Hkv:
+        raise ValueError(f"mtlflashattn_amd: k has {Hkv} heads, v {vs[h_axis]}")
+    if ks[s_axis] != vs[s_axis]:
         raise ValueError("mtlflashattn_amd: k/v seqlen mismatch")
 
 
@@ -262,7 +267,9 @@ def _run(q, k, v, out, *, scale, causal, softcap, window_left, window_right, ali
                 p.softmax_lse = lse.data_ptr()
             if paged is not None:
                 p.block_table = block_table.data_ptr()
-            p.varlen_no_single_rows = 1 if (varlen and no_single_rows) else 0
+            if varlen and no_single_rows:
+                p.varlen_no_single_rows = 1
+            p.workspace = ent[2]
             _launch(p, ent[1], q.device)
             return out
     if Dp != D:  # the kernels read 16-byte chunks: zero-pad the head dim
@@ -323,7 +330,8 @@ def _fits_strides(x: torch.Tensor) -> bool:
 
 def _prepare(q, k, v, out, batch, Hq, Hkv, Lq, Lk, Dp, varlen, scale, causal, softcap, window_left, window_right,
              has_alibi, alibi_bstride, lse_strides=None, paged=None):
-    """(parameter template without data pointers, split-KV choice) of a call."""
+    """(parameter template without data pointers, split-KV choice, its
+    workspace bytes) of a call."""
     p = _hip.MfaFwdParams()
     p.q = p.k = p.v = p.o = 256  # placeholders: the choice below reads no tensor
     p.q_batch_stride, p.q_seq_stride, p.q_head_stride = _strides_bsh(q)
@@ -351,8 +359,9 @@ def _prepare(q, k, v, out, batch, Hq, Hkv, Lq, Lk, Dp, varlen, scale, causal, so
     if paged is not None:
         p.block_table_batch_stride, p.page_block_size, p.num_pages = paged
     chunk = _split_choice(p, q.dtype, hint)
+    nbytes = _hip.workspace_bytes(p, chunk) if chunk else 0
     p.q = p.k = p.v = p.o = p.cu_seqlens_q = p.cu_seqlens_k = p.alibi_slopes = None
-    return p, chunk
+    return p, chunk, nbytes
 
 
 def _split_choice(p, dtype, hint):
@@ -382,11 +391,18 @@ def _launch(p, chunk, device):
     if chunk:
         # split-KV: partials in a workspace from torch's stream-ordered
         # caching allocator (reused only after these kernels ran)
-        nbytes = _hip.workspace_bytes(p, chunk)
+        nbytes = _hip.workspace_bytes(p, chunk) if p.workspace is None else p.workspace
         ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
         _hip.fwd_splitkv(p, chunk, ws.data_ptr(), nbytes, stream)
     else:
         _hip.fwd(p, stream)
+
+
+def _device_i32(t, device):
+    """t as a contiguous int32 tensor on `device` (itself when it is one)."""
+    if t.dtype is torch.int32 and t.device == device and t.is_contiguous():
+        return t
+    return t.to(device=device, dtype=torch.int32).contiguous()
 
 
 def _out_dtype(q, out_dtype):
@@ -436,7 +452,7 @@ def flash_attn_forward(q, k, v, scale, causal, softcap=0.0, window_left=-1, wind
 
 
 def forward_bshd(q, k, v, scale, causal, softcap=0.0, window_left=-1, window_right=-1,
-                 alibi_slopes=None, out_dtype=None, return_lse=False, packed=None):
+                 alibi_slopes=None, out_dtype=None, return_lse=False, packed=None, checked=False):
     """Heads-third forward: q [B,Lq,Hq,D], k/v [B,Lk,Hkv,D] -> [B,Lq,Hq,D].
 
     Same result as flash_attn_forward on the transposed views followed by
@@ -444,12 +460,14 @@ def forward_bshd(q, k, v, scale, causal, softcap=0.0, window_left=-1, window_rig
     the kernel writes the heads-third output directly (no layout copies).
     return_lse=True returns (out, lse [B,Hq,Lq] fp32).  packed: the tensors
     q, k, v are views of, (q, kv) or (qkv,), as _split_packed takes them.
+    checked: the caller has made the checks of softcap and shapes.
     """
     if _trace_enabled():
         _record_trace(q.dtype, q.shape[-1], q.shape[1], k.shape[1], causal)
-    if softcap < 0:
-        raise ValueError("mtlflashattn_amd: softcap must be >= 0 (0 disables capping)")
-    _check_qkv_shapes(q, k, v, h_axis=2, s_axis=1)
+    if not checked:
+        if softcap < 0:
+            raise ValueError("mtlflashattn_amd: softcap must be >= 0 (0 disables capping)")
+        _check_qkv_shapes(q, k, v, h_axis=2, s_axis=1)
     B, Lq, Hq, D = q.shape
     if _needs_grad(q, k, v) and _out_dtype(q, out_dtype) == q.dtype:
         _alibi_arg(alibi_slopes, B, Hq, q.device)  # validate before autograd records anything
@@ -500,8 +518,7 @@ def forward_varlen(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap=0.0
         return (o, lse) if return_lse else o
     out = torch.empty(q.shape, dtype=_out_dtype(q, out_dtype), device=q.device)
     lse = torch.empty(Hq, q.shape[0], dtype=torch.float32, device=q.device) if return_lse else None
-    cu_q = cu_q.to(device=q.device, dtype=torch.int32).contiguous()
-    cu_k = cu_k.to(device=q.device, dtype=torch.int32).contiguous()
+    cu_q, cu_k = _device_i32(cu_q, q.device), _device_i32(cu_k, q.device)
     if block_table is not None:
         block_table = block_table.to(device=q.device, dtype=torch.int32)
         if block_table.stride(1) != 1:
@@ -519,7 +536,11 @@ def forward_varlen(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap=0.0
 
 
 def _needs_grad(*tensors):
-    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+    if torch.is_grad_enabled():
+        for t in tensors:
+            if t.requires_grad:
+                return True
+    return False
 
 
 def _run_bwd(q, k, v, out, dout, lse, *, scale, causal, softcap, window_left, window_right, alibi, alibi_bstride,
@@ -546,55 +567,103 @@ def _run_bwd(q, k, v, out, dout, lse, *, scale, causal, softcap, window_left, wi
         return tuple(torch.zeros(t.shape, dtype=gdt, device=t.device) if g is None else g.zero_()
                      for t, g in zip((q, k, v), into))
     Dp = -(-D // 8) * 8
+    device = q.device
     ts = [q, k, v, out, dout.to(q.dtype)]
-    if Dp != D:
-        ts = [F.pad(t, (0, Dp - D)) for t in ts]
-    q_, k_, v_, o_, do_ = (_abi_operand(t) for t in ts)
+    lse = lse.contiguous()
+    if dlse is not None:
+        dlse = dlse.to(device=device, dtype=torch.float32).contiguous()
+    # launch parameters of this signature (everything but the data pointers),
+    # prepared once; tensors used in place
+    key = ent = None
+    if Dp == D:
+        key = (*((t.shape, t.stride()) for t in ts), *((None if g is None else g.stride()) for g in into), q.dtype, gdt,
+               device.index, float(scale), bool(causal), float(softcap), int(window_left), int(window_right),
+               alibi is not None, alibi_bstride, (cu_q.shape[0], Lq, Lk) if varlen else None, lse.stride())
+        ent = _bwd_plans.get(key)
+    ptrs = [t.data_ptr() for t in ts]
     # (a padded head dim, or a view the library cannot address: through a tensor of its own)
-    dq, dk, dv = (torch.empty(t.shape, dtype=gdt, device=q.device) if g is None or Dp != D or not _fits_abi(g) else g
-                  for t, g in zip((q_, k_, v_), into))
-
-    bp = _hip.MfaBwdParams()
+    grads = [torch.empty(t.shape[:-1] + (Dp,), dtype=gdt, device=device) if g is None or Dp != D or not _fits_abi(g) else g
+             for t, g in zip(ts, into)]
+    in_place = all(g is None or g is t for g, t in zip(into, grads))
+    if ent is None or not in_place or (ptrs[0] | ptrs[1] | ptrs[2] | ptrs[3] | ptrs[4]) & 15:
+        if Dp != D:
+            ts = [F.pad(t, (0, Dp - D)) for t in ts]
+        given, ts = ts, [_abi_operand(t) for t in ts]
+        ptrs = [t.data_ptr() for t in ts]
+        # (a copy in an operand's or a gradient's place has other strides than the signature)
+        if not in_place or any(x is not y for x, y in zip(given, ts)):
+            key = None
+        ent = _prepare_bwd(ts, grads, gdt, batch, Hq, Hkv, Lq, Lk, Dp, varlen, scale, causal, softcap, window_left,
+                           window_right, alibi_bstride if alibi is not None else None, lse)
+        if key is not None:
+            if len(_bwd_plans) >= _PLANS_MAX:
+                _bwd_plans.clear()
+            _bwd_plans[key] = ent
+    template, nbytes = ent
+    bp = _hip.MfaBwdParams.from_buffer_copy(template)
     p = bp.fwd
-    p.q, p.k, p.v, p.o = q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr()
-    p.q_batch_stride, p.q_seq_stride, p.q_head_stride = _strides_bsh(q_)
-    p.k_batch_stride, p.k_seq_stride, p.k_head_stride = _strides_bsh(k_)
-    p.v_batch_stride, p.v_seq_stride, p.v_head_stride = _strides_bsh(v_)
-    p.o_batch_stride, p.o_seq_stride, p.o_head_stride = _strides_bsh(o_)
-    p.batch, p.heads_q, p.heads_kv = batch, Hq, Hkv
-    p.seqlen_q, p.seqlen_k, p.head_dim = Lq, Lk, Dp
+    p.q, p.k, p.v, p.o, bp.dout = ptrs
+    dq, dk, dv = grads
+    bp.dq, bp.dk, bp.dv = dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
+    p.softmax_lse = lse.data_ptr()
     if varlen:
         p.cu_seqlens_q, p.cu_seqlens_k = cu_q.data_ptr(), cu_k.data_ptr()
-    p.scale, p.softcap = float(scale), float(softcap)
-    p.window_left, p.window_right = int(window_left), int(window_right)
-    p.causal = 1 if causal else 0
     if alibi is not None:
         p.alibi_slopes = alibi.data_ptr()
-        p.alibi_batch_stride = alibi_bstride
-    p.dtype_in = p.dtype_out = _hip.DTYPE_CODES[q.dtype]
-    lse = lse.contiguous()
-    p.softmax_lse = lse.data_ptr()
     if dlse is not None:
-        dlse = dlse.to(device=q.device, dtype=torch.float32).contiguous()
         bp.dlse = dlse.data_ptr()
-    p.lse_batch_stride, p.lse_head_stride = (0, lse.stride(0)) if varlen else (lse.stride(0), lse.stride(1))
-    bp.dout = do_.data_ptr()
-    bp.do_batch_stride, bp.do_seq_stride, bp.do_head_stride = _strides_bsh(do_)
-    bp.dq = dq.data_ptr()
-    bp.dq_batch_stride, bp.dq_seq_stride, bp.dq_head_stride = _strides_bsh(dq)
-    bp.dk = dk.data_ptr()
-    bp.dk_batch_stride, bp.dk_seq_stride, bp.dk_head_stride = _strides_bsh(dk)
-    bp.dv = dv.data_ptr()
-    bp.dv_batch_stride, bp.dv_seq_stride, bp.dv_head_stride = _strides_bsh(dv)
-    bp.dtype_grad = _hip.DTYPE_CODES[gdt]
-    device = q.device
-    with torch.cuda.device(device):
-        nbytes = _hip.bwd_workspace_bytes(bp)
-        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-        _hip.bwd(bp, ws.data_ptr(), nbytes, torch._C._cuda_getCurrentRawStream(device.index))
+    _launch_bwd(bp, nbytes, device)
     if Dp != D:
         dq, dk, dv = dq[..., :D], dk[..., :D], dv[..., :D]
     return tuple(t if g is None or g is t else g.copy_(t) for t, g in zip((dq, dk, dv), into))
+
+
+# prepared backward launch parameters per call signature (see _run_bwd)
+_bwd_plans = {}
+
+
+def _prepare_bwd(ts, grads, gdt, batch, Hq, Hkv, Lq, Lk, Dp, varlen, scale, causal, softcap, window_left, window_right,
+                 alibi_bstride, lse):
+    """(parameter template without data pointers, workspace bytes) of a
+    backward call on the tensors ts = [q, k, v, out, dout] into grads."""
+    q, k, v, o, do = ts
+    bp = _hip.MfaBwdParams()
+    p = bp.fwd
+    p.q_batch_stride, p.q_seq_stride, p.q_head_stride = _strides_bsh(q)
+    p.k_batch_stride, p.k_seq_stride, p.k_head_stride = _strides_bsh(k)
+    p.v_batch_stride, p.v_seq_stride, p.v_head_stride = _strides_bsh(v)
+    p.o_batch_stride, p.o_seq_stride, p.o_head_stride = _strides_bsh(o)
+    p.batch, p.heads_q, p.heads_kv = batch, Hq, Hkv
+    p.seqlen_q, p.seqlen_k, p.head_dim = Lq, Lk, Dp
+    p.scale, p.softcap = float(scale), float(softcap)
+    p.window_left, p.window_right = int(window_left), int(window_right)
+    p.causal = 1 if causal else 0
+    p.dtype_in = p.dtype_out = _hip.DTYPE_CODES[q.dtype]
+    p.lse_batch_stride, p.lse_head_stride = (0, lse.stride(0)) if varlen else (lse.stride(0), lse.stride(1))
+    bp.do_batch_stride, bp.do_seq_stride, bp.do_head_stride = _strides_bsh(do)
+    bp.dq_batch_stride, bp.dq_seq_stride, bp.dq_head_stride = _strides_bsh(grads[0])
+    bp.dk_batch_stride, bp.dk_seq_stride, bp.dk_head_stride = _strides_bsh(grads[1])
+    bp.dv_batch_stride, bp.dv_seq_stride, bp.dv_head_stride = _strides_bsh(grads[2])
+    bp.dtype_grad = _hip.DTYPE_CODES[gdt]
+    # placeholders: sizing the workspace reads no tensor
+    p.q = p.k = p.v = p.o = p.softmax_lse = bp.dout = bp.dq = bp.dk = bp.dv = 256
+    if varlen:
+        p.cu_seqlens_q = p.cu_seqlens_k = 256
+    if alibi_bstride is not None:
+        p.alibi_slopes = 256
+        p.alibi_batch_stride = alibi_bstride
+    nbytes = _hip.bwd_workspace_bytes(bp)
+    p.alibi_slopes = p.cu_seqlens_q = p.cu_seqlens_k = None
+    return bp, nbytes
+
+
+def _launch_bwd(bp, nbytes, device):
+    idx = device.index
+    if idx != torch.cuda.current_device():
+        with torch.cuda.device(device):
+            return _launch_bwd(bp, nbytes, device)
+    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
+    _hip.bwd(bp, ws.data_ptr(), nbytes, torch._C._cuda_getCurrentRawStream(idx))
 
 
 # Inputs of the autograd functions as the caller holds them: (q, k, v), (q, kv)
@@ -660,8 +729,7 @@ class _FlashAttnVarlenFn(torch.autograd.Function):
                                   no_single_rows=no_single_rows)
         batch, Hq = cu_q.shape[0] - 1, q.shape[1]
         alibi, bstride = _alibi_arg(alibi_slopes, batch, Hq, q.device)
-        cu_q = cu_q.to(device=q.device, dtype=torch.int32).contiguous()
-        cu_k = cu_k.to(device=q.device, dtype=torch.int32).contiguous()
+        cu_q, cu_k = _device_i32(cu_q, q.device), _device_i32(cu_k, q.device)
         ctx.save_for_backward(out, lse, cu_q, cu_k, *ts)
         ctx.cfg = dict(scale=scale, causal=causal, softcap=softcap, window_left=window_left,
                        window_right=window_right, alibi=alibi, alibi_bstride=bstride, seqlen_q=max_q,

@@ -70,3 +70,31 @@ def test_one_input_needs_a_gradient_and_empty_batches():
         assert torch.equal(g, both[i])
     (g,) = grad(mfa.flash_attn_qkvpacked_func, [rand(0, 20, 3, 4, 64, dtype=torch.bfloat16)], dout[:0])
     assert g.shape == (0, 20, 3, 4, 64)
+
+
+def test_prepared_parameters_follow_layout_and_alignment():
+    # the same shapes again as other views: gradients are those of contiguous copies
+    torch.manual_seed(1)
+    shape = (2, 40, 4, 64)
+    q, k, v, dout = (rand(*shape, dtype=torch.bfloat16) for _ in range(4))
+    ref = grad(mfa.flash_attn_func, [q, k, v], dout)
+
+    def off(t):  # contiguous, 2 bytes past an aligned address
+        b = torch.empty(t.numel() + 8, dtype=t.dtype, device=DEV)[1:1 + t.numel()].view(t.shape)
+        return b.copy_(t)
+
+    def strided(t):
+        b = torch.empty(*t.shape[:-1], 72, dtype=t.dtype, device=DEV)[..., :64]
+        return b.copy_(t)
+
+    def heads_second(t):
+        return t.transpose(1, 2).contiguous().transpose(1, 2)
+
+    for change in (off, strided, heads_second):
+        for i in range(4):
+            ts = [q, k, v, dout]
+            ts[i] = change(ts[i])
+            got = grad(mfa.flash_attn_func, ts[:3], ts[3])
+            assert all(torch.equal(a, b) for a, b in zip(got, ref)), (change.__name__, i)
+    again = grad(mfa.flash_attn_func, [q, k, v], dout)
+    assert all(torch.equal(a, b) for a, b in zip(again, ref))
