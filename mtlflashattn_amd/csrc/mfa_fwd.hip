@@ -2229,12 +2229,7 @@ KernelCfg cfg32s(const char* name, bool paged) {
 // tile configuration per (dtype, padded head dim, bias)
 // Tile shape per padded head dim: QB 32-query blocks per wavefront, NKB
 // 32-key blocks per K/V block (overridable at build time for tuning sweeps).
-#ifndef MFA_D32_TILE
-#define MFA_D32_TILE 2, 2
-#endif
-#ifndef MFA_D64_TILE
-#define MFA_D64_TILE 2, 2
-#endif
+// (head dims up to 64 have two heights, see prefer_rows128)
 #ifndef MFA_D96_TILE
 #define MFA_D96_TILE 1, 2
 #endif
@@ -2261,7 +2256,7 @@ KernelCfg cfg32s(const char* name, bool paged) {
 #endif
 // paged K/V (block_table) runs on the 256-row and fp32 kernels only
 template <bool IS_BF16, bool BIAS>
-KernelCfg select16(int dp, bool fills_chip, bool paged, bool pp256) {
+KernelCfg select16(int dp, bool fills_chip, bool paged, bool pp256, bool rows128) {
     if (MFA_PINGPONG && fills_chip && dp == 128)  // one 32-row query block per wavefront
         return cfg16pp<128, 1, 2, IS_BF16, BIAS>(IS_BF16 ? "mfa_fwd16pp<bf16,d128,1,2>" : "mfa_fwd16pp<f16,d128,1,2>");
     if (MFA_PINGPONG && fills_chip && dp <= 64 && pp256) {  // one 32-row query block per wavefront
@@ -2282,14 +2277,18 @@ KernelCfg select16(int dp, bool fills_chip, bool paged, bool pp256) {
         return cfg16pp<64, 2, 2, IS_BF16, BIAS>(IS_BF16 ? "mfa_fwd16pp<bf16,d64,2,2>" : "mfa_fwd16pp<f16,d64,2,2>");
     }
     switch (dp) {
-        case 32: return cfg16<32, MFA_D32_TILE, IS_BF16, BIAS>(IS_BF16 ? "mfa_fwd16<bf16,d32," MFA_STR(MFA_D32_TILE) ">" : "mfa_fwd16<f16,d32," MFA_STR(MFA_D32_TILE) ">", paged);
+        case 32:
+            if (rows128)
+                return cfg16<32, 1, 2, IS_BF16, BIAS>(IS_BF16 ? "mfa_fwd16<bf16,d32,1, 2>" : "mfa_fwd16<f16,d32,1, 2>", paged);
+            return cfg16<32, 2, 2, IS_BF16, BIAS>(IS_BF16 ? "mfa_fwd16<bf16,d32,2, 2>" : "mfa_fwd16<f16,d32,2, 2>", paged);
         case 64:
             // with a bias two query blocks per wavefront exceed the register
             // budget and spill to scratch inside the loop (2.2-2.8x slower)
-            if constexpr (BIAS)
-                return cfg16<64, 1, 2, IS_BF16, BIAS>(IS_BF16 ? "mfa_fwd16<bf16,d64,1, 2>" : "mfa_fwd16<f16,d64,1, 2>", paged);
-            else
-                return cfg16<64, MFA_D64_TILE, IS_BF16, BIAS>(IS_BF16 ? "mfa_fwd16<bf16,d64," MFA_STR(MFA_D64_TILE) ">" : "mfa_fwd16<f16,d64," MFA_STR(MFA_D64_TILE) ">", paged);
+            if constexpr (!BIAS) {
+                if (!rows128)
+                    return cfg16<64, 2, 2, IS_BF16, BIAS>(IS_BF16 ? "mfa_fwd16<bf16,d64,2, 2>" : "mfa_fwd16<f16,d64,2, 2>", paged);
+            }
+            return cfg16<64, 1, 2, IS_BF16, BIAS>(IS_BF16 ? "mfa_fwd16<bf16,d64,1, 2>" : "mfa_fwd16<f16,d64,1, 2>", paged);
         case 96: return cfg16<96, MFA_D96_TILE, IS_BF16, BIAS>(IS_BF16 ? "mfa_fwd16<bf16,d96," MFA_STR(MFA_D96_TILE) ">" : "mfa_fwd16<f16,d96," MFA_STR(MFA_D96_TILE) ">", paged);
         default: return cfg16<128, MFA_D128_TILE, IS_BF16, BIAS>(IS_BF16 ? "mfa_fwd16<bf16,d128," MFA_STR(MFA_D128_TILE) ">" : "mfa_fwd16<f16,d128," MFA_STR(MFA_D128_TILE) ">", paged);
     }
@@ -2373,6 +2372,50 @@ bool prefer_pp256(const mfa_fwd_params* p, int cus) {
     if (p->cu_seqlens_q || (!p->causal && p->window_left < 0 && p->window_right < 0)) return false;
     if (p->seqlen_q > (1 << 20)) return false;  // (bounds the estimate's loop; long rows balance anyway)
     return tile_makespan(p, 256, 0.545, cus) < 0.9 * tile_makespan(p, 512, 1.0, cus);
+}
+
+// Height of the 4-wavefront tiles at head dims up to 64: 256 rows (two 32-row
+// query blocks per wavefront, each K/V fragment read from LDS once for both)
+// or 128 (one).  The tall tile has the lower cost per row where nothing of it
+// is wasted, but it holds half as many wavefronts per CU and walks the keys of
+// the union of its rows.  128 rows where the tall tiles would do >= 6% more
+// work -- padding of the last tile, and the keys a causal or windowed tile
+// walks for rows that don't see them -- or make fewer than 2 (3 at head dims
+// up to 32) workgroups per CU.  Measured (bf16 D=64, 256 -> 128 rows, us),
+// work: causal H=16 B=16 L=1024 67 -> 62, B=64 L=256 40 -> 35; L=100 B=300
+// H=16 90 -> 52, L=384 H=512 42 -> 34; window (256,256) L=8192 H=16 46 -> 42;
+// 64 varlen lengths in [64, 1024] 227 -> 212, causal 154 -> 136; below 6% it
+// turns: causal L=2048 H=256 208 -> 215, packed B=16 L=1024 Hq=32 Hkv=8
+// causal 106 -> 112.  Grid, non-causal: L=197 B=32 H=12 19.6 -> 16.5, L=2048
+// H=16 54 -> 39, split-KV 128 rows on 65536 keys H=16 88 -> 66; L=768 H=128
+// (384 tiles) 37 -> 33; from 512 tiles L=512 H=256 30 -> 31, H=512 53 -> 58,
+// L=256 H=1536 50 -> 54, 8 varlen lengths in [256, 4096] 241 -> 254.  D=32
+// keeps gaining to 768 tiles (L=512 H=384 33.0 -> 31.1) and ties or loses on
+// long rows above (L=768 H=512 81 -> 85).
+double tile_keys(const mfa_fwd_params* p, double span, double lq, double lk) {
+    const double c = lk - 0.5 * lq;  // mean key position of a row's diagonal
+    double lo = 0., hi = lk;
+    if (p->window_left >= 0) lo = std::max(lo, c - 0.5 * span - p->window_left);
+    if (p->causal) hi = std::min(hi, c + 0.5 * span);
+    else if (p->window_right >= 0) hi = std::min(hi, c + 0.5 * span + p->window_right);
+    return std::max(hi - lo, 64.);
+}
+bool prefer_rows128(const mfa_fwd_params* p, int dp, int pack, int split_keys, int cus) {
+    if (p->heads_kv <= 0) return false;
+    const int64_t units = (int64_t)p->batch * p->heads_q / pack, rows = (int64_t)p->seqlen_q * pack;
+    const int64_t splits = split_keys > 0 ? (p->seqlen_k + (int64_t)split_keys - 1) / split_keys : 1;
+    const int64_t t256 = (rows + 255) / 256, t128 = (rows + 127) / 128;
+    // (the grid bound of make_plan, whose counts the shorter tile doubles)
+    if ((double)units * pack * t128 * std::max<int64_t>(splits, 1) > 0x3fffffff) return false;
+    if (units * t256 * splits < (dp <= 32 ? 3 : 2) * (int64_t)cus) return true;
+    double lq = p->seqlen_q, lk = p->seqlen_k, r256 = t256 * 256., r128 = t128 * 128.;
+    if (p->cu_seqlens_q) {  // only the longest length is known: half of it, half a tile empty
+        lq *= 0.5;
+        lk *= 0.5;
+        r256 = lq * pack + 128.;
+        r128 = lq * pack + 64.;
+    }
+    return r256 * tile_keys(p, 256. / pack, lq, lk) >= 1.06 * r128 * tile_keys(p, 128. / pack, lq, lk);
 }
 
 // ---- Chip geometry: compute units and XCDs of the device a call runs on,
@@ -2779,6 +2822,10 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
     // Lq=26136 Lk=5 H=16: see the design notes)
     const bool tiny_keys = MFA_TK && p->tile_hint == MFA_TILE_AUTO && din != MFA_DTYPE_F32 && !paged &&
                            !single_call && split_keys == 0 && p->seqlen_k <= 32 && p->seqlen_q >= MFA_TK_MIN_ROWS;
+    const int group = p->heads_kv > 0 ? p->heads_q / p->heads_kv : 1;
+    const int pack4 = MFA_4W_HEAD_PACK && !paged && split_keys == 0 && (group == 2 || group == 4) ? group : 1;
+    const bool rows128 = p->tile_hint == MFA_TILE_AUTO && dp <= 64 && !fills_chip &&
+                         prefer_rows128(p, dp, pack4, split_keys, geom.cus);
     const bool split32 = din == MFA_DTYPE_F32 && prefer_split32(p, dp, geom.cus);
     if (din == MFA_DTYPE_F32)
         plan->cfg = bias ? select32<true>(dp, split32, paged) : select32<false>(dp, split32, paged);
@@ -2789,11 +2836,11 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
     else if (tiny_keys)
         plan->cfg = bias ? select16tk<false, true>(dp) : select16tk<false, false>(dp);
     else if (din == MFA_DTYPE_BF16)
-        plan->cfg = bias ? select16<true, true>(dp, fills_chip, paged, pp256)
-                         : select16<true, false>(dp, fills_chip, paged, pp256);
+        plan->cfg = bias ? select16<true, true>(dp, fills_chip, paged, pp256, rows128)
+                         : select16<true, false>(dp, fills_chip, paged, pp256, rows128);
     else
-        plan->cfg = bias ? select16<false, true>(dp, fills_chip, paged, pp256)
-                         : select16<false, false>(dp, fills_chip, paged, pp256);
+        plan->cfg = bias ? select16<false, true>(dp, fills_chip, paged, pp256, rows128)
+                         : select16<false, false>(dp, fills_chip, paged, pp256, rows128);
 
     KArgs& a = plan->args;
     memset(&a, 0, sizeof(a));
