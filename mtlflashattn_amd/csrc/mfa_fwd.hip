@@ -2510,13 +2510,16 @@ int64_t decode_group(int64_t units, int64_t nmax, int dp, bool varlen, int cus) 
 // fp32: the key-split kernel (32-row workgroups) or the 128-row one.  The
 // 128-row tiles are cheaper per pair where they fill the chip, but come in few
 // and unequal pieces: their time is estimated as whole rounds of one tile per CU
-// (equal tiles) or max(heaviest tile, total / CUs), the split's as total / CUs
-// over 32-row tiles times 1.2 (1.3 above head dim 64, where its LDS leaves one
-// wavefront per SIMD).  Measured (us, 128-row -> split): D=64 B=1 L=512 H=2 48.4
-// -> 15.2, B=2 L=1024 H=8 causal 89.8 -> 34.1, B=3 L=1024 H=16 187 -> 145, but
-// B=32 L=200 H=8 56.0 -> 65.9; D=128 B=2 L=1024 H=16 causal 159 -> 122, B=1
-// L=3000 H=16 892 -> 807, but B=3 L=1024 H=16 causal 160 -> 182 and B=4 L=2000
-// H=8 613 -> 736.
+// (equal tiles) or max(heaviest tile, total / CUs) in 32-key blocks; the
+// split's as total / CUs over its 32-row tiles, each 5 blocks longer than its
+// walk (its wavefronts' merge), times 1.1 (1.35 above head dim 64, where its LDS
+// leaves one wavefront per SIMD).  Over 100 shapes of B <= 64, L in [32, 2900]
+// it takes the slower kernel for three, by <= 4%.  Measured (us, 128-row ->
+// split): D=64 B=1 L=512 H=2 48.4 -> 15.2, B=2 L=1024 H=8 causal 89.8 -> 34.1,
+// B=3 L=1024 H=16 187 -> 145, but B=32 L=200 H=8 56.0 -> 65.9 and B=16 L=256
+// H=16 causal 53 -> 69; D=128 B=2 L=1024 H=16 causal 159 -> 122, B=1 L=3000
+// H=16 892 -> 807, but B=3 L=1024 H=16 causal 160 -> 182, B=13 L=299 H=16 172
+// -> 197 and B=34 L=672 H=8 causal 469 -> 530.
 bool prefer_split32(const mfa_fwd_params* p, int dp, int cus) {
     if (p->seqlen_q > (1 << 14)) return false;  // (bounds the loops; long rows fill the chip)
     const int64_t dq = (int64_t)p->seqlen_k - p->seqlen_q;
@@ -2535,7 +2538,7 @@ bool prefer_split32(const mfa_fwd_params* p, int dp, int cus) {
     const double whole = heaviest * tiles[0] == total[0]
                              ? (double)((units * tiles[0] + cus - 1) / cus) * heaviest
                              : std::max((double)heaviest, (double)units * total[0] / cus);
-    return whole > (dp <= 64 ? 1.2 : 1.3) * units * total[1] / (4.0 * cus);
+    return whole > (dp <= 64 ? 1.1 : 1.35) * units * (total[1] + 5 * tiles[1]) / (4.0 * cus);
 }
 
 KernelCfg single_cfg(int dp, bool bf16, int lds) {

@@ -63,7 +63,8 @@ def test_paged_and_ragged_equal_dense():
 
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("B,L,H,causal,split", [(2, 300, 8, True, True), (40, 256, 8, False, False),
-                                                (8, 1000, 16, True, False), (3, 700, 4, False, True)])
+                                                (8, 1000, 16, True, False), (3, 700, 4, False, True),
+                                                (16, 256, 16, True, False)])
 def test_both_sides_of_the_rule(d, B, L, H, causal, split):
     q, k, v = make_qkv(B, L, L, H, H, d, F32, seed=L)
     assert (b"split" in kernel(q, k, causal=causal)) == split
