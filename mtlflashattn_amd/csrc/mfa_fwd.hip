@@ -2759,25 +2759,21 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
             return set_err(MFA_ERR_UNSUPPORTED, "mfa_fwd: ping-pong tiles do not take a block_table");
         fills_chip = false;
     }
-    // Dense calls (no window, no bias) of rows >= 1024 whose 512-row tiles do
-    // not fill the chip but whose 256-row ping-pong tiles do: those tiles (measured 15-25%
-    // faster than the 4-wavefront kernel at D=64: causal B=1 L=4096 H=16 101
-    // -> 80 us, B=1 L=8192 H=8 187 -> 146; non-causal B=1 L=4096 H=16 100 ->
-    // 83, B=1 L=8192 H=8 188 -> 156).
-    // Shorter rows (2-3 tiles of 256) take those tiles too when they make
-    // 3/4 to one round of workgroups (bf16 H=8, 4-wavefront vs ping-pong:
-    // D=64 B=12 L=512 18.2 vs 16.7 us, B=16 L=512 18.8 vs 17.3, B=10 L=768
-    // 24.0 vs 21.9, causal B=16 L=512 21.3 vs 18.4; D=32 B=16 L=512 causal
-    // 17.7 vs 16.1; just past one round they lose: D=64 B=18 L=512 25.1 vs
-    // 30.4, B=11 L=768 33.5 vs 39.6).
+    // Dense calls (no window, no bias) whose 512-row tiles do not fill the chip:
+    // the 256-row ping-pong tiles where they make one round of workgroups, 3/4
+    // full or more (4-wavefront kernel at prefer_rows128's height vs ping-pong,
+    // bf16 D=64: H=8 L=8192 188 vs 173 us, H=40 L=1500 39.8 vs 36.8, H=16 L=4096
+    // 92.6 vs 89.2, H=128 L=512 18.7 vs 17.9; D=32 H=16 L=4096 75.7 vs 68.1).
+    // From there to a round and a half their second round is mostly empty, and
+    // the 4-wavefront kernel runs (H=20 L=4096 121 vs 161, causal 73 vs 84, H=96
+    // L=1024 38 vs 50, causal 27 vs 36, H=12 L=8192 causal 144 vs 159, D=32 H=20
+    // L=4096 97 vs 104).  Above that, rows of >= 4 tiles take them.
     const int64_t t256 = rows256 / 256, n256 = units * t256;
     const bool one_round = t256 >= 2 && 4 * n256 >= 3 * (int64_t)geom.cus && n256 <= geom.cus &&
                            4 * rows256 <= 5 * (int64_t)p->seqlen_q;
     if (p->tile_hint == MFA_TILE_AUTO && !fills_chip && !paged && split_keys == 0 && dp <= 64 &&
         din != MFA_DTYPE_F32 && !bias && !p->cu_seqlens_q && p->window_left < 0 && p->window_right < 0 &&
-        ((n256 >= geom.cus && t256 >= 4) || one_round)) {
-        // (rows of >= 4 tiles over more rounds: shorter rows, e.g. B=64
-        // L=256 H=16, run 40 vs 50 us on the 4-wavefront kernel)
+        ((t256 >= 4 && (n256 == geom.cus || 2 * n256 > 3 * (int64_t)geom.cus)) || one_round)) {
         fills_chip = true;
         pp256 = true;
     } else if (p->tile_hint == MFA_TILE_AUTO && fills_chip && dp <= 64 && din != MFA_DTYPE_F32) {

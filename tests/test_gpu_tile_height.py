@@ -27,6 +27,8 @@ def name(B, L, H, Hk, d, **kw):
     (64, 512, 16, 16, True, 128),    # a causal tile of 256 walks 1/5 more keys
     (16, 2048, 16, 16, True, 256),   # 1/17 more
     (16, 1024, 32, 8, True, 256),    # 4 heads in a tile: 64 positions
+    (1, 4096, 20, 20, False, 128),   # 320 tiles: a quarter past one round
+    (5, 1024, 16, 16, True, 128),
 ])
 def test_rule(monkeypatch, d, B, L, H, Hk, causal, rows):
     if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
