@@ -125,6 +125,10 @@ __device__ __forceinline__ float sum_halves(float x) {
     auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(x), __float_as_int(x), false, false);
     return __int_as_float(sw[0]) + __int_as_float(sw[1]);
 }
+// 2^(from - to) for integer-valued references from <= to (0 for from = -inf)
+__device__ __forceinline__ float pow2_diff(float from, float to) {
+    return __builtin_ldexpf(1.f, (int)fmaxf(from - to, -300.f));
+}
 
 // Direct-to-LDS load (buffer_load_dwordx4 ... lds): lane i of the wave
 // writes the 16 bytes at `off` of the resource to dst + 16*i bytes (dst is

@@ -40,10 +40,6 @@ __device__ __forceinline__ void wait_vm() {
 }
 __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-// 2^(from - to) for integer-valued references from <= to (0 for from = -inf)
-__device__ __forceinline__ float pow2_diff(float from, float to) {
-    return __builtin_ldexpf(1.f, (int)fmaxf(from - to, -300.f));
-}
 // max over the four 16-lane groups (each lane of a group is one query column)
 __device__ __forceinline__ float max_groups(float x) {
     auto a = __builtin_amdgcn_permlane16_swap(__float_as_int(x), __float_as_int(x), false, false);

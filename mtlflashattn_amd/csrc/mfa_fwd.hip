@@ -77,6 +77,11 @@ constexpr int kWaves = 4;
 #ifndef MFA_RESCALE_TAU
 #define MFA_RESCALE_TAU 1
 #endif
+// fp32 probabilities may exceed their reference by far (2^8) without losing
+// bits, and every class of a row's keys starts a reference of its own
+#ifndef MFA_RESCALE_TAU32
+#define MFA_RESCALE_TAU32 8
+#endif
 // padding (elements) of the row-major V tile in LDS
 #ifndef MFA_V_PAD
 #define MFA_V_PAD 32
@@ -299,6 +304,40 @@ __device__ __forceinline__ bool qb_update(RowState& rs, float mx, float c, float
         rs.l *= alpha;
     }
     return moved;
+}
+
+// The fp32 kernels' sums.  A row's 32-key blocks fall into kClasses32 classes by
+// key position (block index modulo the count).  Each class has a softmax state
+// of its own, and the classes' states are added in class order (add_class32).
+// mfa_fwd32s_kernel gives every class a wavefront, mfa_fwd32_kernel walks the
+// classes one after the other: the same bits, so a row does not show which
+// kernel the size of the whole call chose.  Exponent references are whole
+// numbers (ceil(m c)), so every rescale is by a power of two, exact.
+template <int DP>
+constexpr int kClasses32 = DP <= 64 ? 8 : 4;  // (what 160 KB of LDS hold as wavefronts of mfa_fwd32s_kernel)
+__device__ __forceinline__ float ref32(const RowState& rs) { return rs.m == -INFINITY ? -INFINITY : rs.mu; }
+// qb_update with whole-number references
+__device__ __forceinline__ bool qb_update32(RowState& rs, float mx, float c, float tau_c, float& alpha) {
+    alpha = 1.f;
+    const bool moved = __any(mx > rs.thr);
+    if (moved) {
+        const float from = ref32(rs);
+        rs.m = fmax_nn(rs.m, mx);
+        rs.mu = rs.m == -INFINITY ? 0.f : __builtin_ceilf(rs.m * c);
+        rs.thr = rs.m + tau_c;
+        alpha = pow2_diff(from, rs.mu);
+        rs.l *= alpha;
+    }
+    return moved;
+}
+// The next class (reference mw, row sum lw) into the total (mt, lt); its O is
+// added as fma(o, e1, total * e0).
+__device__ __forceinline__ void add_class32(float& mt, float& lt, float mw, float lw, float& e0, float& e1) {
+    const float mn = fmax_nn(mt, mw);
+    e0 = pow2_diff(mt, mn);
+    e1 = pow2_diff(mw, mn);
+    lt = fmaf(lw, e1, lt * e0);
+    mt = mn;
 }
 
 template <int DB>
@@ -1818,11 +1857,22 @@ mfa_fwd16_tk_kernel(KArgs a) {
 // chip; mfa_fwd32s_kernel below serves the others).  K-slot layout of
 // the 32x32x2 MFMA: lane (half, x) supplies k = half, so QK^T step s uses
 // d = s + half*DP/2 and PV step r uses the key held in accumulator register r.
+// The key blocks are walked class by class (kClasses32), with a second set of
+// O accumulators for the sum of the classes before.  Two wavefronts per SIMD up
+// to head dim 96, four at 32 (the registers allow it; one above).  Measured (us,
+// one state for all keys at one wavefront per SIMD -> this): D=64 B=32 L=200
+// H=8 55.1 -> 42.9, B=1 L=4096 H=16 682 -> 570; D=96 B=13 L=299 H=16 131 -> 116;
+// D=128 B=2 L=4096 H=16 causal 1265 -> 1264, B=1 L=3000 H=16 891 -> 893; where
+// a walk has few blocks the additions show: D=128 B=64 L=100 H=16 121 -> 130,
+// B=13 L=299 H=16 167 -> 173, D=32 B=32 L=200 H=8 24.2 -> 25.4.
 template <int DP, int NKB, bool BIAS, bool PAGED>
-__global__ void __launch_bounds__(kThreads) mfa_fwd32_kernel(KArgs a) {
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DP <= 32 ? 4 : DP <= 96 ? 2 : 1)))
+mfa_fwd32_kernel(KArgs a) {
     constexpr int QB = 1;
     constexpr int BM = kWaves * 32;
     constexpr int BN = NKB * 32;
+    constexpr int NC = kClasses32<DP>;
+    static_assert(NKB == 1, "a key block is a class's unit");
     constexpr int DH = DP / 2;   // d values per half-wave
     constexpr int DB = DP / 32;
     constexpr int KST = DP + 4;  // K / Q row stride (floats)
@@ -1886,13 +1936,16 @@ __global__ void __launch_bounds__(kThreads) mfa_fwd32_kernel(KArgs a) {
     rs[0].hi = key_hi(a, rs[0].center, Lk);
     rs[0].slope = a.alibi ? a.alibi[b * a.alibi_bstride + hq] : 0.f;
     row_reset(rs[0]);
-    f32x16_t o[QB][DB];
+    // this class's O and state (rs), and the total of the classes before
+    f32x16_t o[QB][DB], ot[QB][DB];
+    float mt = -INFINITY, lt[QB] = {0.f};
+    bool fresh = true;  // the class has no block yet (wave-uniform)
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[0][db][r] = 0.f;
+        for (int r = 0; r < 16; ++r) o[0][db][r] = ot[0][db][r] = 0.f;
     const float c = BIAS ? kLog2e : a.scale_log2;
-    const float tau_c = (float)MFA_RESCALE_TAU / c;
+    const float tau_c = (float)MFA_RESCALE_TAU32 / c;
 
     const int qlast = min(q0 + BM, Lq) - 1;
     const int klo = key_lo(a, q0 + dq);
@@ -1954,7 +2007,8 @@ __global__ void __launch_bounds__(kThreads) mfa_fwd32_kernel(KArgs a) {
         }
         qb_transform<NKB, BIAS, MASKED, true>(a, sacc, rs[0], j, half);
         float alpha;
-        if (qb_update(rs[0], qb_max<NKB>(sacc), c, tau_c, alpha)) scale_rows<DB>(o[0], alpha);
+        if (qb_update32(rs[0], qb_max<NKB>(sacc), c, tau_c, alpha) && !fresh) scale_rows<DB>(o[0], alpha);
+        fresh = false;
         qb_probs32<NKB>(sacc, rs[0].l, rs[0].mu, c);
 #pragma unroll
         for (int db = 0; db < DB; ++db)
@@ -1967,15 +2021,48 @@ __global__ void __launch_bounds__(kThreads) mfa_fwd32_kernel(KArgs a) {
                 }
     };
 
+    // the end of a class: its state and O into the total
+    auto end_class = [&]() {
+        if (fresh) return;
+        const float mw = ref32(rs[0]);
+        float e0, e1;
+        const bool moved = __any(mw > mt);  // (else e0 = 1 wherever the total is not 0)
+        add_class32(mt, lt[0], mw, sum_halves(rs[0].l), e0, e1);
+        if (moved) scale_rows<DB>(ot[0], e0);
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                ot[0][db][r] = fmaf(o[0][db][r], e1, ot[0][db][r]);
+                o[0][db][r] = 0.f;
+            }
+        row_reset(rs[0]);
+        fresh = true;
+    };
+
+    // block `it` of the tile's range is of class (jbeg / BN + it) % NC
+    const int b0 = jbeg / BN;
+    int cls = 0, it = -b0 & (NC - 1);
+    auto next_class = [&](int& k, int& i) {  // past the classes that have no block (left)
+        while (i >= nblk && k < NC - 1) {
+            ++k;
+            i = (k - b0) & (NC - 1);
+        }
+    };
+    next_class(cls, it);
     if (nblk > 0) {
-        gload(jbeg);
+        gload(jbeg + it * BN);
         swrite(0);
     }
-    for (int it = 0; it < nblk; ++it) {
+    for (int n = 0; n < nblk;) {
+      bool last;
+      do {
         const int j = jbeg + it * BN;
-        const int buf = it & 1;
-        const bool more = it + 1 < nblk;
-        if (more) gload(j + BN);
+        const int buf = n & 1;
+        const bool more = n + 1 < nblk;
+        int ncls = cls, nit = it + NC;
+        next_class(ncls, nit);
+        if (more) gload(jbeg + nit * BN);
         __syncthreads();
 
         const bool skip = !wave_live || (j + BN - 1 < w_lo_first) || (j > w_hi_last);
@@ -1988,18 +2075,25 @@ __global__ void __launch_bounds__(kThreads) mfa_fwd32_kernel(KArgs a) {
             else
                 block(std::false_type{}, kbuf, vbuf, j);
         }
+        last = ncls != cls || !more;
         if (more) swrite(buf ^ 1);
+        cls = ncls;
+        it = nit;
+        ++n;
+      } while (!last);
+      end_class();
     }
 
     // fp32 output (out_f32 is implied for fp32 input)
-    store_out<QB, DB, true>(a, sv, o, rs, wq0, lane, c);
+    rs[0].mu = mt;
+    store_out_l<QB, DB, true>(a, sv, ot, rs, lt, wq0, lane, c);
     if constexpr (BIAS) {
         // the lse of the unshifted ALiBi scores (qb_transform's PRECISE form)
         if (a.alibi && sv.lse && half == 0) {
 #pragma unroll
             for (int qb = 0; qb < QB; ++qb) {
                 const int qrow = wq0 + 32 * qb + l32;
-                if (qrow < sv.Lq) sv.lse[qrow] -= rs[qb].slope * (float)row_dmin(rs[qb]);
+                if (qrow < sv.Lq) sv.lse[qrow] = fmaf(-rs[qb].slope, (float)row_dmin(rs[qb]), sv.lse[qrow]);
             }
         }
     }
@@ -2007,9 +2101,9 @@ __global__ void __launch_bounds__(kThreads) mfa_fwd32_kernel(KArgs a) {
 
 // ----------------------------------------------------------------------------
 // fp32 kernel (v_mfma_f32_32x32x2_f32): 32 query rows per workgroup (lane =
-// query, as in the 16-bit kernels), NW wavefronts that take every NW-th 32-key
-// block, each with its own K and V tile in LDS and its own running softmax, no
-// barrier until their states are merged at the end.  Bound by the matrix pipe:
+// query, as in the 16-bit kernels), NW wavefronts that take one class of 32-key
+// blocks each (kClasses32), with their own K and V tile in LDS and their own
+// softmax, no barrier until their states are added at the end.  Bound by the matrix pipe:
 // a 32 x 32 block is DP MFMAs of 64 cycles against ~250 vector instructions,
 // and re-reading K/V for every 32 rows costs 4 bytes per cycle and wavefront.
 // The split over keys rather than rows is for the grids and walks: 128-row
@@ -2039,10 +2133,11 @@ mfa_fwd32s_kernel(KArgs a) {
     float* kt = k_s[wave];
     float* vt = v_s[wave];
 
-    // key blocks any row of the tile sees; this wavefront's are wave, wave + NW, ...
+    // key blocks any row of the tile sees; this wavefront's are those of its class
     const int klo = key_lo(a, q0 + dq), khi = key_hi(a, q0 + nrow - 1 + dq, Lk);
     const int jbeg = (klo / BN) * BN;
     const int nblk = khi >= klo ? (khi - jbeg) / BN + 1 : 0;
+    const int it0 = (wave - jbeg / BN) & (NW - 1);
     auto load_k = [&](int it) {
         const int j = jbeg + BN * it;
         bool ok;
@@ -2055,9 +2150,9 @@ mfa_fwd32s_kernel(KArgs a) {
         const int64_t off = kv_block_off<PAGED>(a, sv, j, Lk, a.vb, a.vs, ok);
         T::load(vt, reinterpret_cast<const float*>(sv.v) + off, a.vs, ok ? min(BN, Lk - j) : 0, D, lane, false);
     };
-    if (wave < nblk) {
-        load_k(wave);
-        load_v(wave);
+    if (it0 < nblk) {
+        load_k(it0);
+        load_v(it0);
     }
     float qf[DP / 2];
     row_operand<DP>(qf, reinterpret_cast<const float*>(sv.q) + (int64_t)row * a.qs, row < Lq, D, half);
@@ -2078,10 +2173,10 @@ mfa_fwd32s_kernel(KArgs a) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
     const float c = BIAS ? kLog2e : a.scale_log2;
-    const float tau_c = (float)MFA_RESCALE_TAU / c;
+    const float tau_c = (float)MFA_RESCALE_TAU32 / c;
     const int lo_last = key_lo(a, q0 + nrow - 1 + dq), hi_first = key_hi(a, q0 + dq, Lk);
 
-    for (int it = wave; it < nblk; it += NW) {
+    for (int it = it0; it < nblk; it += NW) {
         const bool more = it + NW < nblk;
         const int j = jbeg + BN * it;
         f32x16_t s[1];
@@ -2096,7 +2191,7 @@ mfa_fwd32s_kernel(KArgs a) {
         else
             qb_transform<1, BIAS, true, true>(a, s, rs, j, half);
         float alpha;
-        if (qb_update(rs, qb_max<1>(s), c, tau_c, alpha)) scale_rows<DB>(o, alpha);
+        if (qb_update32(rs, qb_max<1>(s), c, tau_c, alpha)) scale_rows<DB>(o, alpha);
         qb_probs32<1>(s, rs.l, rs.mu, c);
         if (more)
             wait_vm<T::N>();
@@ -2111,26 +2206,23 @@ mfa_fwd32s_kernel(KArgs a) {
     T::put(vt, o, l32, half);
     const float lsum = sum_halves(rs.l);
     if (half == 0) {
-        m_s[wave][l32] = rs.m == -INFINITY ? -INFINITY : rs.mu;
+        m_s[wave][l32] = ref32(rs);
         l_s[wave][l32] = lsum;
     }
     __syncthreads();
     for (int cc = tid; cc < BM * T::CPR; cc += NW * 64) {
         const int r = cc / T::CPR, col = ((cc % T::CPR) ^ T::swz(r)) * 4;
         if (r >= nrow) continue;
-        float m = m_s[0][r];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) m = fmax_nn(m, m_s[w][r]);
-        float x[4] = {0.f, 0.f, 0.f, 0.f}, l = 0.f;
+        float x[4] = {0.f, 0.f, 0.f, 0.f}, m = -INFINITY, l = 0.f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            const float mw = m_s[w][r], e = mw == -INFINITY ? 0.f : fast_exp2(mw - m);
+            float e0, e1;
+            add_class32(m, l, m_s[w][r], l_s[w][r], e0, e1);
             const float4 y = *reinterpret_cast<const float4*>(v_s[w] + cc * 4);
-            x[0] = fmaf(y.x, e, x[0]);
-            x[1] = fmaf(y.y, e, x[1]);
-            x[2] = fmaf(y.z, e, x[2]);
-            x[3] = fmaf(y.w, e, x[3]);
-            l = fmaf(l_s[w][r], e, l);
+            x[0] = fmaf(y.x, e1, x[0] * e0);
+            x[1] = fmaf(y.y, e1, x[1] * e0);
+            x[2] = fmaf(y.z, e1, x[2] * e0);
+            x[3] = fmaf(y.w, e1, x[3] * e0);
         }
         const float inv = l > 0.f ? 1.f / l : 0.f;
         typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4v_t;
@@ -2146,7 +2238,7 @@ mfa_fwd32s_kernel(KArgs a) {
                     t.center = q0 + r + dq;
                     t.lo = key_lo(a, t.center);
                     t.hi = key_hi(a, t.center, Lk);
-                    lse -= rs.slope * (float)row_dmin(t);
+                    lse = fmaf(-rs.slope, (float)row_dmin(t), lse);
                 }
             }
             sv.lse[q0 + r] = lse;
@@ -2220,7 +2312,7 @@ KernelCfg cfg32(const char* name, bool paged) {
 
 template <int DP, bool BIAS>
 KernelCfg cfg32s(const char* name, bool paged) {
-    constexpr int NW = DP <= 64 ? 8 : 4;  // (what 160 KB of LDS hold)
+    constexpr int NW = kClasses32<DP>;
     return KernelCfg{paged ? (kernel_fn)mfa_fwd32s_kernel<DP, NW, BIAS, true>
                            : (kernel_fn)mfa_fwd32s_kernel<DP, NW, BIAS, false>,
                      32, 32, NW * (2 * 32 * DP + 64) * 4, name, NW * 64};
@@ -2507,19 +2599,21 @@ int64_t decode_group(int64_t units, int64_t nmax, int dp, bool varlen, int cus) 
     if (nmax <= 2 || (!varlen && fills)) return nmax;
     return units * nmax <= 2 * (int64_t)cus ? 1 : 2;
 }
-// fp32: the key-split kernel (32-row workgroups) or the 128-row one.  The
-// 128-row tiles are cheaper per pair where they fill the chip, but come in few
-// and unequal pieces: their time is estimated as whole rounds of one tile per CU
-// (equal tiles) or max(heaviest tile, total / CUs) in 32-key blocks; the
-// split's as total / CUs over its 32-row tiles, each 5 blocks longer than its
-// walk (its wavefronts' merge), times 1.1 (1.35 above head dim 64, where its LDS
-// leaves one wavefront per SIMD).  Over 100 shapes of B <= 64, L in [32, 2900]
-// it takes the slower kernel for three, by <= 4%.  Measured (us, 128-row ->
-// split): D=64 B=1 L=512 H=2 48.4 -> 15.2, B=2 L=1024 H=8 causal 89.8 -> 34.1,
-// B=3 L=1024 H=16 187 -> 145, but B=32 L=200 H=8 56.0 -> 65.9 and B=16 L=256
-// H=16 causal 53 -> 69; D=128 B=2 L=1024 H=16 causal 159 -> 122, B=1 L=3000
-// H=16 892 -> 807, but B=3 L=1024 H=16 causal 160 -> 182, B=13 L=299 H=16 172
-// -> 197 and B=34 L=672 H=8 causal 469 -> 530.
+// fp32: the key-split kernel (32-row workgroups) or the 128-row one; the same
+// bits.  The 128-row tiles are cheaper per pair where they fill the chip, but
+// come in few and unequal pieces: their time is estimated as whole rounds of one
+// tile per CU (equal tiles) or max(heaviest tile, total / CUs) in 32-key blocks;
+// the split's as total / CUs over its 32-row tiles, each 5 blocks longer than
+// its walk (the sum of its wavefronts), times 1.1 (1.35 above head dim 64, where
+// its LDS leaves one wavefront per SIMD).  Measured (us, 128-row / split): D=64
+// B=1 L=512 H=2 47.1 / 15.4, B=2 L=1024 H=8 causal 87.3 / 34.8, B=3 L=1024 H=16
+// 150 / 146, B=32 L=200 H=8 43.1 / 65.7, B=16 L=256 H=16 causal 37.6 / 66.5;
+// D=128 B=2 L=1024 H=16 causal 159 / 120, B=3 L=1024 H=16 causal 161 / 180, B=13
+// L=299 H=16 173 / 196, B=34 L=672 H=8 causal 480 / 527.  Over 100 shapes of B <=
+// 40, L in [64, 3000] at head dims 32 to 128 it takes the slower kernel by more
+// than 4% for twelve, mostly the 128-row one near the line (B=1 L=3000 H=16 D=128
+// 893 / 803, B=5 L=2343 H=8 D=32 causal 176 / 151, B=18 L=263 H=8 D=32 causal
+// 27.9 / 21.5; the other way B=4 L=1673 H=8 D=64 243 / 269).
 bool prefer_split32(const mfa_fwd_params* p, int dp, int cus) {
     if (p->seqlen_q > (1 << 14)) return false;  // (bounds the loops; long rows fill the chip)
     const int64_t dq = (int64_t)p->seqlen_k - p->seqlen_q;
