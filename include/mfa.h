@@ -219,7 +219,8 @@ int mfa_params_size(void);
  * HBM-bound shapes.  bf16/fp16 only; results meet the same bars as mfa_fwd.
  *
  * mfa_fwd_split_keys: the library's choice for `params`, 0 = use mfa_fwd.
- * It is 2048 when seqlen_q (the longest query for varlen) is at most 256 and
+ * It is 2048 (above 2M keys the next multiple of 256 that makes at most 1024
+ * chunks) when seqlen_q (the longest query for varlen) is at most 256 and
  * seqlen_k exceeds 2048, else 0 (fp32 and forced ping-pong tiles: 0); a
  * dense call with batch > 1 and batch * heads_q >= 512 gets 0 too (the
  * single pass already fills the chip).  For varlen and batch = 1 calls the

@@ -370,16 +370,17 @@ def _split_choice(p, dtype, hint):
     if _SPLIT_KEYS is not None:
         return _SPLIT_KEYS
     chunk = _hip.split_keys(p)
-    if p.seqlen_q == 1 and (chunk or p.seqlen_k <= _SINGLE_ROW_SPLIT * _MAX_SPLITS):
+    if p.seqlen_q == 1 and (chunk or p.seqlen_k <= _SINGLE_ROW_SPLIT):
         # single rows: the library chunks each sequence by its own length,
         # and says through the workspace whether it splits this call
-        return _SINGLE_ROW_SPLIT if _hip.workspace_bytes(p, _SINGLE_ROW_SPLIT) else 0
+        chunk = chunk or _SINGLE_ROW_SPLIT
+        return chunk if _hip.workspace_bytes(p, chunk) else 0
     return chunk
 
 
-# the chunk of a split request for single-row calls (any valid one: theirs is
-# the library's) and the most chunks such a request may imply
-_SINGLE_ROW_SPLIT, _MAX_SPLITS = 2048, 1024
+# the chunk of a split request for single-row calls that the library's choice
+# leaves whole (any valid one: theirs is the library's)
+_SINGLE_ROW_SPLIT = 2048
 
 
 def _launch(p, chunk, device):

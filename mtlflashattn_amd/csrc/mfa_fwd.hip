@@ -3082,7 +3082,9 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
 
 // Split-KV is chosen for decode-like calls: at most 256 query rows per
 // sequence (one or two query tiles) and more keys than one chunk.  The chunk is a constant (2048 keys: on MI355X
-// the best single size over B=1..64, Hq=16..32, Lk=8K..128K decode shapes).
+// the best single size over B=1..64, Hq=16..32, Lk=8K..128K decode shapes) up
+// to the 2M keys that kMaxSplits of them hold, and the next multiple of 256 that
+// holds the keys above.
 // For varlen and B=1 calls the choice depends on the lengths only, so a
 // sequence gets the same chunks alone (dense B=1) or inside a varlen batch
 // and its rows are bit-identical either way.  A dense batch whose
@@ -3090,6 +3092,10 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
 // single pass: there the split's merge and extra workgroups cost ~8%.
 constexpr int kSplitMaxLq = 256;
 constexpr int kSplitKeys = 2048;
+int split_chunk(int Lk) {
+    const int least = (int)(((int64_t)Lk + kMaxSplits - 1) / kMaxSplits);
+    return std::max(kSplitKeys, (least + 255) / 256 * 256);
+}
 int auto_split_keys(const mfa_fwd_params* p, const ChipGeom& geom) {
     const int64_t kSplitMaxUnits = 2 * (int64_t)geom.cus;  // two workgroups per CU
     if (!p || p->dtype_in == MFA_DTYPE_F32 || p->tile_hint == MFA_TILE_PINGPONG ||
@@ -3097,7 +3103,7 @@ int auto_split_keys(const mfa_fwd_params* p, const ChipGeom& geom) {
         return 0;
     if (p->seqlen_q > kSplitMaxLq || p->seqlen_k <= kSplitKeys) return 0;
     if (!p->cu_seqlens_q && p->batch > 1 && (int64_t)p->batch * p->heads_q >= kSplitMaxUnits) return 0;
-    return kSplitKeys;
+    return split_chunk(p->seqlen_k);
 }
 
 // Enqueue a planned split-KV call with its workspace `ws` (plan.ws_bytes

@@ -381,6 +381,21 @@ def test_split_kv_choice(lib):
     assert lib.mfa_fwd_split_keys(None) == 0
 
 
+@pytest.mark.parametrize("lk", [1 << 21, (1 << 21) + 1, (1 << 21) + 256 * 1024, 1 << 30])
+@pytest.mark.parametrize("lq,B,H", [(1, 1, 1), (1, 3, 8), (4, 1, 1), (4, 600, 1), (256, 2, 2)])
+def test_split_kv_choice_is_one_the_library_takes(lib, lk, lq, B, H):
+    # (a launch holds at most 1024 chunks: 2M keys in chunks of 2048)
+    p = good_params(B=1, L=4096, H=H, Hkv=H, D=64)
+    p.batch, p.seqlen_q, p.seqlen_k = B, lq, lk
+    chunk = lib.mfa_fwd_split_keys(ctypes.byref(p))
+    assert chunk % 256 == 0 and (chunk == 0) == (B == 600)
+    if chunk:
+        assert lk / chunk <= 1024 and (chunk == 2048) == (lk <= 1 << 21)
+        assert lib.mfa_fwd_workspace_bytes(ctypes.byref(p), chunk) >= 0, lib.mfa_last_error()
+    if lk < 1 << 30:  # (what the Python launcher asks for)
+        assert _hip.workspace_bytes(p, _kernel._split_choice(p, torch.bfloat16, 0)) >= 0
+
+
 def test_split_kv_workspace_size(lib):
     p = good_params(B=2, L=3000, H=8, Hkv=2, D=64)
     p.seqlen_q = 3

@@ -19,7 +19,7 @@ import torch
 import mtlflashattn_amd as mfa
 from mtlflashattn_amd import _hip, _kernel
 from oracle import chunked
-from gpu_util import REL_16, REL_16_OUT, default_scale, make_qkv, make_varlen, max_err
+from gpu_util import DEV, REL_16, REL_16_OUT, default_scale, make_qkv, make_varlen, max_err
 
 pytestmark = pytest.mark.gpu
 
@@ -154,3 +154,17 @@ def test_library_choice_on_a_decode_shape(dtype):
     assert _hip.split_keys(p) == 2048
     check(q, k, v, "auto split decode")
     check(q, k, v, "auto split decode causal", causal=True)
+
+
+@pytest.mark.parametrize("lq", [1, 3])
+def test_more_keys_than_1024_chunks_of_2048(lq):
+    lk, d = (1 << 21) + 300, 16
+    g = torch.Generator(device=DEV).manual_seed(lq)
+    q = torch.randn(1, lq, 1, d, generator=g, device=DEV).bfloat16()
+    k, v = (torch.randn(1, lk, 1, d, generator=g, device=DEV).bfloat16() for _ in range(2))
+    # (values whose mean is not 0, so that the result does not vanish over so many keys)
+    v += 1
+    out = mfa.flash_attn_func(q, k, v)
+    p = torch.softmax(q[0, :, 0].double() @ k[0, :, 0].double().t() / d ** 0.5, -1)
+    ref = (p @ v[0, :, 0].double()).cpu()
+    assert max_err(out[0, :, 0], ref) <= REL_16_OUT * ref.abs().max().item()
