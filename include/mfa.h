@@ -215,10 +215,15 @@ int mfa_params_size(void);
  * workgroups compute the chunks in parallel into a caller-provided
  * workspace, and a second kernel merges them (log-sum-exp weighting).  No
  * counterpart in the reference, whose Metal kernels run one threadgroup per
- * query tile over all keys; these three calls are the build's addition for
+ * query tile over all keys; these calls are the build's addition for
  * HBM-bound shapes.  bf16/fp16 only; results meet the same bars as mfa_fwd.
  *
- * mfa_fwd_split_keys: the library's choice for `params`, 0 = use mfa_fwd.
+ * mfa_fwd_split_request: the split_keys with which mfa_fwd_splitkv (and a
+ * workspace of mfa_fwd_workspace_bytes) launches `params` fastest, 0 = use
+ * mfa_fwd.  It is mfa_fwd_split_keys, except for sequences of one query row
+ * (seqlen_q = 1): there it is non-zero exactly where a workspace is used (also
+ * at 2048 keys and below, where mfa_fwd_split_keys is 0).
+ * mfa_fwd_split_keys: the chunk of sequences of several query rows, 0 = none.
  * It is 2048 (above 2M keys the next multiple of 256 that makes at most 1024
  * chunks) when seqlen_q (the longest query for varlen) is at most 256 and
  * seqlen_k exceeds 2048, else 0 (fp32 and forced ping-pong tiles: 0); a
@@ -237,6 +242,7 @@ int mfa_params_size(void);
  * split_keys != 0 only offers the workspace (0 bytes where a workgroup per
  * sequence and K/V head walking all chunks is faster), and the results of
  * mfa_fwd and mfa_fwd_splitkv are the same bits.  softmax_lse and block_table work as in mfa_fwd. */
+int32_t mfa_fwd_split_request(const mfa_fwd_params* params);
 int32_t mfa_fwd_split_keys(const mfa_fwd_params* params);
 int64_t mfa_fwd_workspace_bytes(const mfa_fwd_params* params, int32_t split_keys);
 int mfa_fwd_splitkv(const mfa_fwd_params* params, int32_t split_keys, void* workspace, int64_t workspace_bytes,

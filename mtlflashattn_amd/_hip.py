@@ -158,6 +158,8 @@ def load():
         lib.mfa_fwd.argtypes = [ctypes.POINTER(MfaFwdParams), _c_ptr]
         lib.mfa_fwd_launch_info.restype = ctypes.c_int
         lib.mfa_fwd_launch_info.argtypes = [ctypes.POINTER(MfaFwdParams), ctypes.POINTER(MfaLaunchInfo)]
+        lib.mfa_fwd_split_request.restype = _c_i32
+        lib.mfa_fwd_split_request.argtypes = [ctypes.POINTER(MfaFwdParams)]
         lib.mfa_fwd_split_keys.restype = _c_i32
         lib.mfa_fwd_split_keys.argtypes = [ctypes.POINTER(MfaFwdParams)]
         lib.mfa_fwd_workspace_bytes.restype = ctypes.c_int64
@@ -219,6 +221,11 @@ def fwd(params: MfaFwdParams, stream: int) -> None:
     rc = lib.mfa_fwd(ctypes.byref(params), _c_ptr(stream))
     if rc != MFA_OK:
         raise HipLibraryError(lib.mfa_last_error().decode(errors="replace") or f"mfa_fwd failed ({rc})")
+
+
+def split_request(params: MfaFwdParams) -> int:
+    """The split_keys of this call's fastest launch (0: mfa_fwd)."""
+    return int(load().mfa_fwd_split_request(ctypes.byref(params)))
 
 
 def split_keys(params: MfaFwdParams) -> int:

@@ -55,7 +55,7 @@ def _pp_head_dim_ok(D: int) -> bool:
     """The ping-pong tiles exist for head dims padded to 32, 64 and 128 (not 96)."""
     return -(-D // 32) * 32 != 96
 # Split-KV chunk in keys for bf16/fp16 calls: None = the library's choice
-# (mfa_fwd_split_keys), 0 = never split, a multiple of 64 = that chunk
+# (mfa_fwd_split_request), 0 = never split, a multiple of 64 = that chunk
 # (tests and tuning).
 _SPLIT_KEYS = None
 
@@ -367,20 +367,7 @@ def _prepare(q, k, v, out, batch, Hq, Hkv, Lq, Lk, Dp, varlen, scale, causal, so
 def _split_choice(p, dtype, hint):
     if dtype == torch.float32 or hint in _PP_HINTS:
         return 0
-    if _SPLIT_KEYS is not None:
-        return _SPLIT_KEYS
-    chunk = _hip.split_keys(p)
-    if p.seqlen_q == 1 and (chunk or p.seqlen_k <= _SINGLE_ROW_SPLIT):
-        # single rows: the library chunks each sequence by its own length,
-        # and says through the workspace whether it splits this call
-        chunk = chunk or _SINGLE_ROW_SPLIT
-        return chunk if _hip.workspace_bytes(p, chunk) else 0
-    return chunk
-
-
-# the chunk of a split request for single-row calls that the library's choice
-# leaves whole (any valid one: theirs is the library's)
-_SINGLE_ROW_SPLIT = 2048
+    return _hip.split_request(p) if _SPLIT_KEYS is None else _SPLIT_KEYS
 
 
 def _launch(p, chunk, device):

@@ -3105,6 +3105,19 @@ int auto_split_keys(const mfa_fwd_params* p, const ChipGeom& geom) {
     if (!p->cu_seqlens_q && p->batch > 1 && (int64_t)p->batch * p->heads_q >= kSplitMaxUnits) return 0;
     return split_chunk(p->seqlen_k);
 }
+// The request that gives a call its fastest launch: auto_split_keys, and for
+// sequences of one query row (whose chunks plan_decode takes from their own
+// lengths) any valid chunk wherever their partials would use a workspace.
+int split_request(const mfa_fwd_params* p, const ChipGeom& geom) {
+    const int chunk = auto_split_keys(p, geom);
+    if (!p || p->seqlen_q != 1 || p->seqlen_k <= 0 || p->dtype_in == MFA_DTYPE_F32 ||
+        p->tile_hint == MFA_TILE_PINGPONG || p->tile_hint == MFA_TILE_PINGPONG256)
+        return chunk;
+    const int any = split_chunk(p->seqlen_k);
+    Plan plan;
+    if (make_plan(p, &plan, geom, any) != MFA_OK) return chunk;  // (the call itself says why)
+    return plan.ws_bytes > 0 ? any : 0;
+}
 
 // Enqueue a planned split-KV call with its workspace `ws` (plan.ws_bytes
 // bytes, 256-byte aligned): the chunk kernel writes every partial the merge
@@ -3215,6 +3228,11 @@ int mfa_fwd_launch_info(const mfa_fwd_params* params, mfa_launch_info* info) {
 }
 
 int32_t mfa_fwd_split_keys(const mfa_fwd_params* params) { return auto_split_keys(params, chip_geometry_current()); }
+
+int32_t mfa_fwd_split_request(const mfa_fwd_params* params) {
+    g_err[0] = 0;
+    return split_request(params, chip_geometry_current());
+}
 
 int64_t mfa_fwd_workspace_bytes(const mfa_fwd_params* params, int32_t split_keys) {
     g_err[0] = 0;

@@ -396,6 +396,32 @@ def test_split_kv_choice_is_one_the_library_takes(lib, lk, lq, B, H):
         assert _hip.workspace_bytes(p, _kernel._split_choice(p, torch.bfloat16, 0)) >= 0
 
 
+def test_split_request_covers_single_rows(lib):
+    # a caller of the C ABI gets a single-row call's workspace from the request
+    # alone: non-zero exactly where the launch uses one
+    def req(Lq=1, Lk=2000, B=1, H=8, Hkv=8, D=64, **kw):
+        p = good_params(B=B, L=4096, H=H, Hkv=Hkv, D=D, dtype=kw.pop("dtype", _hip.MFA_DTYPE_BF16))
+        p.seqlen_q, p.seqlen_k = Lq, Lk
+        for f, val in kw.items():
+            setattr(p, f, val)
+        r = lib.mfa_fwd_split_request(ctypes.byref(p))
+        n = lib.mfa_fwd_workspace_bytes(ctypes.byref(p), r)
+        assert n >= 0
+        return r, n, lib.mfa_fwd_split_keys(ctypes.byref(p))
+    for kw in (dict(), dict(B=6, Lk=1500), dict(H=32, D=128), dict(Lk=2048, cu_seqlens_q=256, cu_seqlens_k=256)):
+        r, n, k = req(**kw)
+        assert r > 0 and n > 0 and k == 0, kw
+    for kw in (dict(Lk=512), dict(Lk=1), dict(Lk=0), dict(B=64, H=16, Hkv=16, Lk=4096), dict(B=600, Lk=4096)):
+        assert req(**kw)[:2] == (0, 0), kw  # one workgroup walks the keys
+    assert req(Lk=5000)[0] == 2048 and req(Lk=5000)[1] > 0
+    for kw in (dict(Lq=4, Lk=2000), dict(Lq=4, Lk=5000), dict(Lq=257, Lk=5000), dict(Lq=4, Lk=5000, B=600)):
+        r, _, k = req(**kw)
+        assert r == k, kw  # several rows: the choice of mfa_fwd_split_keys
+    for kw in (dict(dtype=_hip.MFA_DTYPE_F32), dict(tile_hint=_hip.MFA_TILE_PINGPONG)):
+        assert req(**kw)[0] == 0, kw
+    assert lib.mfa_fwd_split_request(None) == 0
+
+
 def test_split_kv_workspace_size(lib):
     p = good_params(B=2, L=3000, H=8, Hkv=2, D=64)
     p.seqlen_q = 3
