@@ -222,7 +222,11 @@ int mfa_params_size(void);
  * workspace of mfa_fwd_workspace_bytes) launches `params` fastest, 0 = use
  * mfa_fwd.  It is mfa_fwd_split_keys, except for sequences of one query row
  * (seqlen_q = 1): there it is non-zero exactly where a workspace is used (also
- * at 2048 keys and below, where mfa_fwd_split_keys is 0).
+ * at 2048 keys and below, where mfa_fwd_split_keys is 0).  For a varlen call
+ * that may mix such sequences with longer ones (varlen_no_single_rows 0) and
+ * whose longer ones are not split, it is a chunk of seqlen_k keys or more
+ * wherever the single rows would use a workspace: the longer ones then run as
+ * in mfa_fwd.
  * mfa_fwd_split_keys: the chunk of sequences of several query rows, 0 = none.
  * It is 2048 (above 2M keys the next multiple of 256 that makes at most 1024
  * chunks) when seqlen_q (the longest query for varlen) is at most 256 and
@@ -241,7 +245,10 @@ int mfa_params_size(void);
  * library, from their own key count, in every entry point alike: there
  * split_keys != 0 only offers the workspace (0 bytes where a workgroup per
  * sequence and K/V head walking all chunks is faster), and the results of
- * mfa_fwd and mfa_fwd_splitkv are the same bits.  softmax_lse and block_table work as in mfa_fwd. */
+ * mfa_fwd and mfa_fwd_splitkv are the same bits.  In a call that mixes them with
+ * longer sequences their partials follow the longer ones' in the workspace; a
+ * workspace of the longer ones' size (as reported with varlen_no_single_rows 1)
+ * is taken too, the single rows are then not split.  softmax_lse and block_table work as in mfa_fwd. */
 int32_t mfa_fwd_split_request(const mfa_fwd_params* params);
 int32_t mfa_fwd_split_keys(const mfa_fwd_params* params);
 int64_t mfa_fwd_workspace_bytes(const mfa_fwd_params* params, int32_t split_keys);

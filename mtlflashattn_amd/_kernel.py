@@ -211,7 +211,8 @@ def _strides_bsh(x: torch.Tensor):
 
 
 def _run(q, k, v, out, *, scale, causal, softcap, window_left, window_right, alibi, alibi_bstride,
-         cu_q=None, cu_k=None, seqlen_q=None, seqlen_k=None, lse=None, block_table=None, no_single_rows=False):
+         cu_q=None, cu_k=None, seqlen_q=None, seqlen_k=None, lse=None, block_table=None, no_single_rows=False,
+         short_single_rows=False):
     """Launch the HIP forward on [B, S, H, D] views q, k, v and write `out`.
 
     out: [B, Sq, Hq, D] tensor of q.dtype or float32 (full-precision output).
@@ -224,6 +225,8 @@ def _run(q, k, v, out, *, scale, causal, softcap, window_left, window_right, ali
     count comes from seqlen_k (dense) or cu_k (varlen).
     no_single_rows: (varlen) no sequence has exactly one query row, so the
     single-row launch for such sequences is skipped.
+    short_single_rows: (varlen) such sequences have few keys, so no workspace is
+    taken to split them.
     """
     _kernel_mode()
     B, Sq, Hq, D = q.shape
@@ -248,11 +251,12 @@ def _run(q, k, v, out, *, scale, causal, softcap, window_left, window_right, ali
         key = (q.shape, q.stride(), k.shape, k.stride(), v.shape, v.stride(), out.shape, out.stride(), q.dtype,
                out.dtype, q.device.index, float(scale), bool(causal), float(softcap), int(window_left),
                int(window_right), alibi is not None, alibi_bstride,
-               (cu_q.shape[0], Lq, Lk) if varlen else None, _TILE_HINT, _SPLIT_KEYS, lse_strides, paged)
+               (cu_q.shape[0], Lq, Lk, no_single_rows, short_single_rows) if varlen else None, _TILE_HINT, _SPLIT_KEYS, lse_strides, paged)
         ent = _plans.get(key)
         if ent is None and all(_fits_strides(t) for t in (q, k, v, out)):
             ent = _prepare(q, k, v, out, batch, Hq, Hkv, Lq, Lk, Dp, varlen, scale, causal, softcap, window_left,
-                           window_right, alibi is not None, alibi_bstride, lse_strides, paged)
+                           window_right, alibi is not None, alibi_bstride, lse_strides, paged,
+                           no_single_rows or short_single_rows)
             if len(_plans) >= _PLANS_MAX:
                 _plans.clear()
             _plans[key] = ent
@@ -267,8 +271,8 @@ def _run(q, k, v, out, *, scale, causal, softcap, window_left, window_right, ali
                 p.softmax_lse = lse.data_ptr()
             if paged is not None:
                 p.block_table = block_table.data_ptr()
-            if varlen and no_single_rows:
-                p.varlen_no_single_rows = 1
+            if varlen and not no_single_rows:
+                p.varlen_no_single_rows = 0
             p.workspace = ent[2]
             _launch(p, ent[1], q.device)
             return out
@@ -308,12 +312,22 @@ def _run(q, k, v, out, *, scale, causal, softcap, window_left, window_right, ali
     if paged is not None:
         p.block_table = block_table.data_ptr()
         p.block_table_batch_stride, p.page_block_size, p.num_pages = paged
+    p.varlen_no_single_rows = 1 if (varlen and (no_single_rows or short_single_rows)) else 0
+    chunk = _split_choice(p, q.dtype, hint)
+    p.workspace = _hip.workspace_bytes(p, chunk) if chunk else 0
     p.varlen_no_single_rows = 1 if (varlen and no_single_rows) else 0
-    _launch(p, _split_choice(p, q.dtype, hint), q.device)
+    _launch(p, chunk, q.device)
     if dst is not out:
         out.copy_(dst[..., :D])
     return out
 
+
+# Single rows over at most this many keys, beside longer rows, are walked by one
+# workgroup per K/V head: up to two of the library's 256-key chunks they are in
+# any case, and up to four the merge's launch costs what the split saves (bf16
+# Hq=32 Hkv=8 D=128, a 512-row prefill beside 31 rows of 64 to 1024 keys: 72.3 us
+# walked, 74.8 split; beside 31 of 256 to 4096 keys 119 and 111).
+SHORT_SINGLE_ROW_KEYS = 1024
 
 # prepared launch parameters per call signature (see _run's fast path)
 _plans = {}
@@ -329,9 +343,10 @@ def _fits_strides(x: torch.Tensor) -> bool:
 
 
 def _prepare(q, k, v, out, batch, Hq, Hkv, Lq, Lk, Dp, varlen, scale, causal, softcap, window_left, window_right,
-             has_alibi, alibi_bstride, lse_strides=None, paged=None):
+             has_alibi, alibi_bstride, lse_strides=None, paged=None, whole_single_rows=False):
     """(parameter template without data pointers, split-KV choice, its
-    workspace bytes) of a call."""
+    workspace bytes) of a call.  whole_single_rows: (varlen) the workspace is
+    sized without single-row sequences; those that there are get none."""
     p = _hip.MfaFwdParams()
     p.q = p.k = p.v = p.o = 256  # placeholders: the choice below reads no tensor
     p.q_batch_stride, p.q_seq_stride, p.q_head_stride = _strides_bsh(q)
@@ -342,6 +357,7 @@ def _prepare(q, k, v, out, batch, Hq, Hkv, Lq, Lk, Dp, varlen, scale, causal, so
     p.seqlen_q, p.seqlen_k, p.head_dim = Lq, Lk, Dp
     if varlen:  # placeholders: the choice below only needs to see varlen
         p.cu_seqlens_q = p.cu_seqlens_k = 256
+        p.varlen_no_single_rows = int(whole_single_rows)
     p.scale, p.softcap = float(scale), float(softcap)
     p.window_left, p.window_right = int(window_left), int(window_right)
     p.causal = 1 if causal else 0
@@ -379,7 +395,7 @@ def _launch(p, chunk, device):
     if chunk:
         # split-KV: partials in a workspace from torch's stream-ordered
         # caching allocator (reused only after these kernels ran)
-        nbytes = _hip.workspace_bytes(p, chunk) if p.workspace is None else p.workspace
+        nbytes = p.workspace
         ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
         _hip.fwd_splitkv(p, chunk, ws.data_ptr(), nbytes, stream)
     else:
@@ -472,7 +488,7 @@ def forward_bshd(q, k, v, scale, causal, softcap=0.0, window_left=-1, window_rig
 
 def forward_varlen(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap=0.0, window_left=-1,
                    window_right=-1, alibi_slopes=None, out_dtype=None, return_lse=False, block_table=None,
-                   _grad=True, no_single_rows=False, packed=None):
+                   _grad=True, no_single_rows=False, short_single_rows=False, packed=None):
     """Packed varlen forward in ONE launch: q [Tq,Hq,D], k/v [Tk,Hkv,D].
 
     cu_q/cu_k: int32 [batch+1] device tensors; max_q/max_k: the longest
@@ -485,7 +501,8 @@ def forward_varlen(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap=0.0
     table, q.dtype output) go through the HIP backward.  no_single_rows: the
     caller knows no sequence has exactly one query row (the library then
     skips the single-row launch for such sequences; a one-row sequence would
-    be left unwritten).  packed: as in forward_bshd.
+    be left unwritten).  short_single_rows: such sequences have at most
+    SHORT_SINGLE_ROW_KEYS keys each.  packed: as in forward_bshd.
     """
     batch = cu_q.shape[0] - 1
     Hq = q.shape[1]
@@ -502,7 +519,8 @@ def forward_varlen(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap=0.0
                                   "run them under torch.no_grad() or without inputs that require grad")
     if _grad and block_table is None and _needs_grad(q, k, v) and _out_dtype(q, out_dtype) == q.dtype:
         o, lse = _FlashAttnVarlenFn.apply(cu_q, cu_k, max_q, max_k, scale, causal, softcap, window_left,
-                                          window_right, alibi_slopes, no_single_rows, *(packed or (q, k, v)))
+                                          window_right, alibi_slopes, no_single_rows, short_single_rows,
+                                          *(packed or (q, k, v)))
         return (o, lse) if return_lse else o
     out = torch.empty(q.shape, dtype=_out_dtype(q, out_dtype), device=q.device)
     lse = torch.empty(Hq, q.shape[0], dtype=torch.float32, device=q.device) if return_lse else None
@@ -514,7 +532,7 @@ def forward_varlen(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap=0.0
     _run(q[None], k if block_table is not None else k[None], v if block_table is not None else v[None], out[None],
          scale=scale, causal=causal, softcap=softcap, window_left=window_left, window_right=window_right,
          alibi=alibi, alibi_bstride=bstride, cu_q=cu_q, cu_k=cu_k, seqlen_q=max_q, seqlen_k=max_k, lse=lse,
-         block_table=block_table, no_single_rows=no_single_rows)
+         block_table=block_table, no_single_rows=no_single_rows, short_single_rows=short_single_rows)
     return (out, lse) if return_lse else out
 
 
@@ -710,11 +728,11 @@ class _FlashAttnVarlenFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, cu_q, cu_k, max_q, max_k, scale, causal, softcap, window_left, window_right, alibi_slopes,
-                no_single_rows, *ts):
+                no_single_rows, short_single_rows, *ts):
         q, k, v = _split_packed(ts)
         out, lse = forward_varlen(q, k, v, cu_q, cu_k, max_q, max_k, scale, causal, softcap, window_left,
                                   window_right, alibi_slopes, return_lse=True, _grad=False,
-                                  no_single_rows=no_single_rows)
+                                  no_single_rows=no_single_rows, short_single_rows=short_single_rows)
         batch, Hq = cu_q.shape[0] - 1, q.shape[1]
         alibi, bstride = _alibi_arg(alibi_slopes, batch, Hq, q.device)
         cu_q, cu_k = _device_i32(cu_q, q.device), _device_i32(cu_k, q.device)
@@ -734,7 +752,7 @@ class _FlashAttnVarlenFn(torch.autograd.Function):
         q, k, v = _split_packed(ts)
         dqkv = _run_bwd(q[None], k[None], v[None], out[None], dout[None], lse, cu_q=cu_q, cu_k=cu_k, dlse=dlse,
                         into=grads and tuple(g[None] for g in _split_packed(grads)), **ctx.cfg)
-        return (None,) * 11 + (grads or tuple(g[0] for g in dqkv))
+        return (None,) * 12 + (grads or tuple(g[0] for g in dqkv))
 
 
 def _plain(*tensors) -> bool:

@@ -2410,10 +2410,11 @@ struct Plan {
     bool empty;
     kernel_fn combine = nullptr;  // split-KV merge kernel
     int64_t ws_bytes = 0;         // split-KV workspace
-    // the single-row kernel: instead of the above (decode_only: every sequence
-    // of the call has one query row; combine is then its merge kernel, for
-    // dec.nsplit > 1), or as a second launch on the single-row sequences of a
-    // varlen call that mixes them with longer ones
+    int64_t dec_bytes = 0;        // its end: the partial results of single rows
+    // the single-row kernel (and, with dec_bytes, its merge kernel): instead of
+    // the above (decode_only: every sequence of the call has one query row), or
+    // beside it on the single-row sequences of a varlen call that mixes them
+    // with longer ones
     bool decode_only = false, decode_too = false;
     DecodeKernels dk;
     DArgs dec;
@@ -2428,6 +2429,7 @@ void launch_plan(const Plan& plan, hipStream_t st) {
         hipLaunchKernelGGL((decode_fn)plan.dk.attend, dim3(plan.dec_grid), dim3(kDecodeThreads), 0, st, plan.dec);
 }
 
+int padded_dim(int D) { return D <= 32 ? 32 : D <= 64 ? 64 : D <= 96 ? 96 : 128; }
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Ping-pong tile height for dense causal / windowed calls, where tiles cost
@@ -2593,6 +2595,12 @@ ChipGeom chip_geometry_current() { return chip_geometry_of(nullptr); }
 //   24 sequences to 4096 (192)            56.7 / 56.0 / 60.7 / 70.2
 //   64 to 4096 (512)                     138.5 / 134.0 / 136.2 / 140.2
 //   48 to 8192, H=16 D=64 (768)          185.9 / 187.3 / 190.2 / 212.7
+// Calls that mix single rows with longer ones count every sequence as a unit
+// (Hq=32 Hkv=8 D=128, us, all chunks in one workgroup -> this rule): 1 and 4 rows
+// in turn over 32K keys, 2 sequences 477 -> 106, 8 639 -> 341; a 2048-row prefill
+// beside 7 rows over 32K keys 486 -> 223, beside 63 of 512 to 8192 350 -> 335; 1
+// and 4 rows in turn, 64 sequences of 256 to 4096 245 -> 228, but of 4096 each
+// 342 -> 356.
 int64_t decode_group(int64_t units, int64_t nmax, int dp, bool varlen, int cus) {
     const int64_t rounds = (units + cus - 1) / cus;
     const bool fills = dp > 64 ? 4 * units >= 3 * cus * rounds : units >= 2 * (int64_t)cus;
@@ -2668,7 +2676,7 @@ int plan_decode(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int d
     // Lk=1500 H=16 D=64, 37 MB, 14.4 -> 15.4).
     d.nt = (int64_t)p->batch * p->seqlen_k * p->heads_kv * p->head_dim * 4 >= ((int64_t)64 << 20) && d.rt <= 2;
     d.ws_ld = dp;
-    plan->ws_bytes = 0;
+    plan->dec_bytes = 0;
     const int64_t nmax = decode_chunks_max(p->seqlen_k);
     if (may_split && nmax > 1) {
         const int64_t rows = nmax * units * d.nr;
@@ -2676,7 +2684,7 @@ int plan_decode(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int d
         if (group < nmax && units * nmax <= 0x7fffffffLL / 2 && rows <= 0x7fffffffLL / 2) {
             d.group = (int32_t)group;
             d.nsplit = (int32_t)((nmax + group - 1) / group);
-            plan->ws_bytes = rows * dp * 4 + (rows * 8 + 255) / 256 * 256;
+            plan->dec_bytes = rows * dp * 4 + (rows * 8 + 255) / 256 * 256;
         }
     }
     plan->dec_grid = (int)(units * d.nsplit);
@@ -2754,7 +2762,7 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
     if (p->k_seq_stride < 0 || p->v_seq_stride < 0 || (kv_span + D) * es >= ((int64_t)1 << 31))
         return set_err(MFA_ERR_INVALID, "mfa_fwd: k/v sequence strides must be >= 0 and span < 2 GiB per 64 rows");
 
-    const int dp = D <= 32 ? 32 : D <= 64 ? 64 : D <= 96 ? 96 : 128;
+    const int dp = padded_dim(D);
     const bool bias = p->softcap > 0.f || p->alibi_slopes != nullptr || !(p->scale > 0.f);
     // the 512-row ping-pong tiles are used when they still give every CU a
     // workgroup (256 CUs on MI355X)
@@ -2836,7 +2844,16 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
         } else
             fills_chip = units * (rows512 / 512) >= geom.cus && 4 * rows512 <= 5 * rows256;
     }
+    // Single rows: a 16-bit call whose every sequence has one query row runs
+    // the single-row kernel, whatever the tile hint.  A varlen call that may
+    // mix such sequences with longer ones runs its kernel on the longer ones
+    // and the single-row kernel on the others (a second launch), so each
+    // sequence's rows are those of its own dense call.
+    const bool single_call = din != MFA_DTYPE_F32 && p->seqlen_q == 1;
+    const bool mixed_rows =
+        din != MFA_DTYPE_F32 && !single_call && p->cu_seqlens_q != nullptr && !p->varlen_no_single_rows;
     bool pp256 = p->tile_hint == MFA_TILE_PINGPONG256;
+    const bool workspace = split_keys != 0;
     if (split_keys != 0) {
         // split-KV runs on the 4-wavefront kernel (bf16/fp16)
         if (split_keys < 0 || split_keys % 64 != 0)
@@ -2845,7 +2862,12 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
         if (din == MFA_DTYPE_F32) return set_err(MFA_ERR_UNSUPPORTED, "mfa_fwd_splitkv: fp32 has no split-KV path");
         if (pp_hint)
             return set_err(MFA_ERR_UNSUPPORTED, "mfa_fwd_splitkv: split-KV uses the 256-row tiles");
-        fills_chip = false;
+        // (one chunk for the longer rows of a mixed call: they are not split,
+        // the workspace is for the single rows)
+        if (mixed_rows && split_keys >= p->seqlen_k)
+            split_keys = 0;
+        else
+            fills_chip = false;
     }
     const bool paged = p->block_table != nullptr;
     if (paged) {
@@ -2901,14 +2923,6 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
         else
             pp256 = prefer_pp256(p, geom.cus);
     }
-    // Single rows: a 16-bit call whose every sequence has one query row runs
-    // the single-row kernel, whatever the tile hint.  A varlen call that may
-    // mix such sequences with longer ones runs its kernel on the longer ones
-    // and the single-row kernel on the others (a second launch), so each
-    // sequence's rows are those of its own dense call.
-    const bool single_call = din != MFA_DTYPE_F32 && p->seqlen_q == 1;
-    const bool mixed_rows =
-        din != MFA_DTYPE_F32 && !single_call && p->cu_seqlens_q != nullptr && !p->varlen_no_single_rows;
     // At most 32 keys per sequence under many query rows (cross-attention to
     // a short conditioning sequence): the tiny-key kernel, which keeps the
     // keys in registers and streams the query rows (measured at bf16 D=128
@@ -2993,10 +3007,11 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
         return set_err(MFA_ERR_INVALID, "mfa_fwd_splitkv: %d chunks of %d keys exceed %d; use larger chunks",
                        (int)((p->seqlen_k + (int64_t)split_keys - 1) / split_keys), split_keys, kMaxSplits);
     if (single_call || mixed_rows) {
-        const int rc = plan_decode(p, plan, geom, dp, bias, split_keys != 0 && single_call);
+        const int rc = plan_decode(p, plan, geom, dp, bias, workspace);
         if (rc != MFA_OK) return rc;
         if (single_call) {
             plan->decode_only = true;
+            plan->ws_bytes = plan->dec_bytes;
             plan->grid = plan->dec_grid;
             plan->cfg.lds = plan->dk.lds;
             if (plan->grid == 0) plan->empty = true;
@@ -3074,10 +3089,21 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
         plan->grid *= a.nsplit;
         const int64_t rows = (int64_t)a.nsplit * a.U * p->seqlen_q;
         plan->ws_bytes = rows * dp * 4 + ((rows * 4 + 255) / 256) * 256;
+        if (plan->dec_bytes) plan->ws_bytes = (plan->ws_bytes + 255) / 256 * 256;
         plan->combine = din == MFA_DTYPE_BF16 ? (kernel_fn)mfa_combine_kernel<true> : (kernel_fn)mfa_combine_kernel<false>;
     }
+    plan->ws_bytes += plan->dec_bytes;
     if (plan->grid == 0) plan->empty = true;
     return MFA_OK;
+}
+// The single rows of a mixed call without their part of the workspace: one
+// workgroup walks each unit's chunks (the same bits).
+void walk_single_rows(Plan* plan) {
+    plan->dec.nsplit = 1;
+    plan->dec.group = INT32_MAX / 2;
+    plan->dec_grid = plan->dec.units;
+    plan->ws_bytes -= plan->dec_bytes;
+    plan->dec_bytes = 0;
 }
 
 // Split-KV is chosen for decode-like calls: at most 256 query rows per
@@ -3107,13 +3133,15 @@ int auto_split_keys(const mfa_fwd_params* p, const ChipGeom& geom) {
 }
 // The request that gives a call its fastest launch: auto_split_keys, and for
 // sequences of one query row (whose chunks plan_decode takes from their own
-// lengths) any valid chunk wherever their partials would use a workspace.
+// lengths) any valid chunk wherever their partials would use a workspace -- one
+// that holds every key where longer rows, not split, stand beside them.
 int split_request(const mfa_fwd_params* p, const ChipGeom& geom) {
     const int chunk = auto_split_keys(p, geom);
-    if (!p || p->seqlen_q != 1 || p->seqlen_k <= 0 || p->dtype_in == MFA_DTYPE_F32 ||
+    if (!p || p->seqlen_q < 1 || p->seqlen_k <= 0 || p->seqlen_k > INT32_MAX - 255 || p->dtype_in == MFA_DTYPE_F32 ||
         p->tile_hint == MFA_TILE_PINGPONG || p->tile_hint == MFA_TILE_PINGPONG256)
         return chunk;
-    const int any = split_chunk(p->seqlen_k);
+    if (p->seqlen_q > 1 && (chunk != 0 || !p->cu_seqlens_q || p->varlen_no_single_rows)) return chunk;
+    const int any = p->seqlen_q > 1 ? (p->seqlen_k + 255) / 256 * 256 : split_chunk(p->seqlen_k);
     Plan plan;
     if (make_plan(p, &plan, geom, any) != MFA_OK) return chunk;  // (the call itself says why)
     return plan.ws_bytes > 0 ? any : 0;
@@ -3124,25 +3152,23 @@ int split_request(const mfa_fwd_params* p, const ChipGeom& geom) {
 // kernel reads (each chunk of each row that exists, lse -inf and O 0 for a
 // chunk without a valid key), so the workspace needs no clearing.
 int launch_splitkv(Plan& plan, void* ws, hipStream_t st, const char* who) {
-    if (plan.decode_only) {
-        DArgs& d = plan.dec;
-        d.ws_o = static_cast<float*>(ws);
-        d.ws_ml = d.ws_o + (int64_t)decode_chunks_max(d.f.Lk) * d.units * d.nr * d.ws_ld;
-        launch_plan(plan, st);
-        if (d.nsplit > 1)
-            hipLaunchKernelGGL((decode_fn)plan.dk.merge, dim3((unsigned)(d.units * d.nr)), dim3(64), 0, st, d);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return set_err(MFA_ERR_LAUNCH, "%s: launch failed: %s", who, hipGetErrorString(e));
-        return MFA_OK;
-    }
     KArgs& a = plan.args;
-    const int64_t rows = (int64_t)a.nsplit * a.U * a.Lq;
-    a.ws_o = static_cast<float*>(ws);
-    a.ws_lse = a.ws_o + rows * a.ws_ld;
+    DArgs& d = plan.dec;
+    if (!plan.decode_only) {
+        const int64_t rows = (int64_t)a.nsplit * a.U * a.Lq;
+        a.ws_o = static_cast<float*>(ws);
+        a.ws_lse = a.ws_o + rows * a.ws_ld;
+    }
+    if (plan.dec_bytes) {
+        d.ws_o = reinterpret_cast<float*>(static_cast<char*>(ws) + (plan.ws_bytes - plan.dec_bytes));
+        d.ws_ml = d.ws_o + (int64_t)decode_chunks_max(d.f.Lk) * d.units * d.nr * d.ws_ld;
+    }
     // one chunk (every key range fits): the kernels store O themselves
     launch_plan(plan, st);
-    if (a.nsplit > 1)
+    if (!plan.decode_only && a.nsplit > 1)
         hipLaunchKernelGGL(plan.combine, dim3((unsigned)((int64_t)a.U * a.Lq)), dim3(64), 0, st, a);
+    if (plan.dec_bytes)
+        hipLaunchKernelGGL((decode_fn)plan.dk.merge, dim3((unsigned)(d.units * d.nr)), dim3(64), 0, st, d);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_err(MFA_ERR_LAUNCH, "%s: launch failed: %s", who, hipGetErrorString(e));
     return MFA_OK;
@@ -3253,6 +3279,9 @@ int mfa_fwd_splitkv(const mfa_fwd_params* params, int32_t split_keys, void* work
     if (plan.empty) return MFA_OK;
     if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
         return set_err(MFA_ERR_INVALID, "mfa_fwd_splitkv: workspace must be a 256-byte aligned device pointer");
+    // (a workspace of the longer rows alone is taken)
+    if (plan.decode_too && workspace_bytes < plan.ws_bytes && workspace_bytes >= plan.ws_bytes - plan.dec_bytes)
+        walk_single_rows(&plan);
     if (workspace_bytes < plan.ws_bytes)
         return set_err(MFA_ERR_INVALID, "mfa_fwd_splitkv: workspace of %lld bytes, %lld needed",
                        (long long)workspace_bytes, (long long)plan.ws_bytes);
@@ -3266,19 +3295,13 @@ int mfa_fwd_splitkv_static(const mfa_fwd_params* params, int32_t split_keys, voi
     const int rc = make_plan(params, &plan, chip_geometry_of(static_cast<hipStream_t>(stream)), split_keys);
     if (rc != MFA_OK) return rc;
     if (plan.empty) return MFA_OK;
-    int64_t need = plan.ws_bytes;
-    if (plan.decode_only) {
-        // single rows: the size of the request's own chunks decides whether
-        // the call is taken; beyond the scratch, a workgroup walks the chunks
-        const mfa_fwd_params* p = params;
-        const int64_t rows = ((int64_t)p->seqlen_k + split_keys - 1) / split_keys * p->batch * p->heads_q;
-        if (need > MFA_STATIC_SCRATCH_BYTES) {
-            plan.dec.nsplit = 1;
-            plan.dec.group = INT32_MAX / 2;
-            plan.dec_grid = plan.dec.units;
-        }
-        need = rows * plan.dec.ws_ld * 4 + (rows * 4 + 255) / 256 * 256;
-    }
+    // the size of the request's own chunks decides whether the call is taken;
+    // single rows whose partials are larger than the scratch walk their chunks
+    const mfa_fwd_params* p = params;
+    const int64_t rows = ((int64_t)p->seqlen_k + split_keys - 1) / split_keys * p->batch * p->heads_q * p->seqlen_q;
+    const int dp = padded_dim(p->head_dim);
+    const int64_t need = rows * dp * 4 + (rows * 4 + 255) / 256 * 256;
+    if (plan.dec_bytes && plan.ws_bytes > MFA_STATIC_SCRATCH_BYTES) walk_single_rows(&plan);
     if (need > MFA_STATIC_SCRATCH_BYTES)
         return set_err(MFA_ERR_INVALID,
                        "mfa_fwd_splitkv_static: this call needs %lld bytes of workspace, more than the static "

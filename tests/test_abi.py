@@ -422,6 +422,45 @@ def test_split_request_covers_single_rows(lib):
     assert lib.mfa_fwd_split_request(None) == 0
 
 
+def test_mixed_calls_have_a_workspace_for_their_single_rows(lib):
+    # a varlen call that may mix single rows with longer ones splits the keys of
+    # its single rows as a call of single rows alone does, beside a main launch
+    # that is split (few query rows) or not
+    def make(Lq, Lk=9000, none=0, **kw):
+        p = good_params(B=5, L=4096, H=8, Hkv=2, D=64, dtype=kw.pop("dtype", _hip.MFA_DTYPE_BF16))
+        p.cu_seqlens_q = p.cu_seqlens_k = 256
+        p.seqlen_q, p.seqlen_k, p.varlen_no_single_rows = Lq, Lk, none
+        for f, val in kw.items():
+            setattr(p, f, val)
+        return p
+
+    def size(p, chunk):
+        n = lib.mfa_fwd_workspace_bytes(ctypes.byref(p), chunk)
+        assert n >= 0, lib.mfa_last_error()
+        return n
+    alone = size(make(1), 2048)
+    assert alone > 0
+    # split main launch: both parts, the single rows' behind the other's
+    p, rest = make(4), make(4, none=1)
+    chunk = lib.mfa_fwd_split_request(ctypes.byref(p))
+    assert chunk == 2048 == lib.mfa_fwd_split_keys(ctypes.byref(p)) == lib.mfa_fwd_split_request(ctypes.byref(rest))
+    main = size(rest, chunk)
+    assert main > 0 and size(p, chunk) == -(-main // 256) * 256 + alone
+    # main launch not split: a request that makes one chunk of every key
+    p, rest = make(2048), make(2048, none=1)
+    chunk = lib.mfa_fwd_split_request(ctypes.byref(p))
+    assert chunk >= 9000 and chunk % 256 == 0 and lib.mfa_fwd_split_request(ctypes.byref(rest)) == 0
+    assert size(p, chunk) == alone
+    # nothing to split: few keys, fp32, ping-pong hints, dense calls
+    for p in (make(2048, Lk=512), make(2048, dtype=_hip.MFA_DTYPE_F32),
+              make(2048, tile_hint=_hip.MFA_TILE_PINGPONG256), make(2048, cu_seqlens_q=None, cu_seqlens_k=None)):
+        assert lib.mfa_fwd_split_request(ctypes.byref(p)) == 0
+    # a workspace too small for the longer rows is still refused
+    p = make(4)
+    assert lib.mfa_fwd_splitkv(ctypes.byref(p), 2048, ctypes.c_void_p(1 << 20), main - 256, None) == _hip.MFA_ERR_INVALID
+    assert b"needed" in lib.mfa_last_error()
+
+
 def test_split_kv_workspace_size(lib):
     p = good_params(B=2, L=3000, H=8, Hkv=2, D=64)
     p.seqlen_q = 3

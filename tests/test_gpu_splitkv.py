@@ -168,3 +168,64 @@ def test_more_keys_than_1024_chunks_of_2048(lq):
     p = torch.softmax(q[0, :, 0].double() @ k[0, :, 0].double().t() / d ** 0.5, -1)
     ref = (p @ v[0, :, 0].double()).cpu()
     assert max_err(out[0, :, 0], ref) <= REL_16_OUT * ref.abs().max().item()
+
+
+@pytest.mark.parametrize("long_rows", [4, 300])
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 128), (4, 4, 64), (34, 2, 40)])
+@pytest.mark.parametrize("paged", [False, True])
+def test_single_rows_of_a_mixed_call(long_rows, hq, hkv, d, paged, monkeypatch):
+    # single rows beside longer ones, which are split (4 rows) or not (300):
+    # their keys are split over workgroups as in a call of their own, and every
+    # sequence has the bits of its own dense call with and without a workspace,
+    # with one of the longer rows alone, and whatever the workspace held before
+    from test_gpu_lse_paged import paginate
+
+    lens_q = [1, long_rows, 1, 1, 0, 1, 2, 1]
+    lens_k = [9000, 5000, 300, 1, 700, 0, 2000, 2600]
+    q, k, v, cu_q, cu_k = make_varlen(lens_q, lens_k, hq, hkv, d, torch.bfloat16, seed=d)
+    args, kw = (cu_q, cu_k, max(lens_q), max(lens_k)), {}
+    pk, pv = k, v
+    if paged:
+        pk, pv, kw["block_table"] = paginate(k, v, lens_k, 256, seed=d)
+    sq, sk = ([0] + torch.tensor(x).cumsum(0).tolist() for x in (lens_q, lens_k))
+
+    def check(out, lse, what):
+        for i, (n, m) in enumerate(zip(lens_q, lens_k)):
+            o, l = out[sq[i]:sq[i + 1]], lse[:, sq[i]:sq[i + 1]]
+            if n and m:
+                a, al = mfa.flash_attn_func_with_lse(q[None, sq[i]:sq[i + 1]], k[None, sk[i]:sk[i + 1]],
+                                                     v[None, sk[i]:sk[i + 1]], causal=True)
+                assert torch.equal(o, a[0]) and torch.equal(l, al[0]), (what, i)
+            elif n:
+                assert (o == 0).all() and torch.isneginf(l).all(), (what, i)
+
+    for poison in (float("nan"), 1e30):
+        junk = torch.full((1 << 24,), poison, device=DEV)
+        del junk
+        check(*mfa.flash_attn_varlen_func_with_lse(q, pk, pv, *args, causal=True, **kw), "workspace")
+    monkeypatch.setattr(_kernel, "SHORT_SINGLE_ROW_KEYS", 1 << 30)
+    check(*mfa.flash_attn_varlen_func_with_lse(q, pk, pv, *args, causal=True, **kw), "workspace of the longer rows")
+    monkeypatch.setattr(_kernel, "_SPLIT_KEYS", 0)
+    check(*mfa.flash_attn_varlen_func_with_lse(q, pk, pv, *args, causal=True, **kw), "walked")
+
+
+def test_single_rows_of_a_mixed_static_call():
+    # the static scratch: single rows whose partials fit behind the longer rows'
+    # are split, others walk; the same bits as with a workspace
+    for n, lk in ((6, 3000), (40, 16000)):
+        lens_q, lens_k = [1, 3] * (n // 2), [lk, 900] * (n // 2)
+        q, k, v, cu_q, cu_k = make_varlen(lens_q, lens_k, 64, 2, 128, torch.bfloat16, seed=n)
+        want = mfa.flash_attn_varlen_func(q, k, v, cu_q, cu_k, 3, lk)
+        out = torch.full_like(q, float("nan"))
+        p = _hip.MfaFwdParams()
+        p.q, p.k, p.v, p.o = (t.data_ptr() for t in (q, k, v, out))
+        p.q_seq_stride, p.q_head_stride = p.o_seq_stride, p.o_head_stride = q.stride()[:2]
+        p.k_seq_stride, p.k_head_stride = p.v_seq_stride, p.v_head_stride = k.stride()[:2]
+        p.cu_seqlens_q, p.cu_seqlens_k = cu_q.data_ptr(), cu_k.data_ptr()
+        p.batch, p.heads_q, p.heads_kv, p.seqlen_q, p.seqlen_k, p.head_dim = n, 64, 2, 3, lk, 128
+        p.scale, p.window_left, p.window_right = default_scale(128), -1, -1
+        p.dtype_in = p.dtype_out = _hip.MFA_DTYPE_BF16
+        chunk = _hip.split_request(p)
+        assert (_hip.workspace_bytes(p, chunk) > 64 << 20) == (n == 40)
+        _hip.fwd_splitkv_static(p, chunk, torch.cuda.current_stream().cuda_stream)
+        assert torch.equal(out, want), n
