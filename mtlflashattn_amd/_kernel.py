@@ -16,6 +16,7 @@ raises RuntimeError.
 from __future__ import annotations
 
 import atexit
+import contextlib
 import os
 import sys
 import warnings
@@ -313,8 +314,7 @@ def _run(q, k, v, out, *, scale, causal, softcap, window_left, window_right, ali
         p.block_table = block_table.data_ptr()
         p.block_table_batch_stride, p.page_block_size, p.num_pages = paged
     p.varlen_no_single_rows = 1 if (varlen and (no_single_rows or short_single_rows)) else 0
-    chunk = _split_choice(p, q.dtype, hint)
-    p.workspace = _hip.workspace_bytes(p, chunk) if chunk else 0
+    chunk, p.workspace = _split_and_workspace(p, q.dtype, hint, q.device)
     p.varlen_no_single_rows = 1 if (varlen and no_single_rows) else 0
     _launch(p, chunk, q.device)
     if dst is not out:
@@ -374,10 +374,24 @@ def _prepare(q, k, v, out, batch, Hq, Hkv, Lq, Lk, Dp, varlen, scale, causal, so
         p.lse_batch_stride, p.lse_head_stride = lse_strides
     if paged is not None:
         p.block_table_batch_stride, p.page_block_size, p.num_pages = paged
-    chunk = _split_choice(p, q.dtype, hint)
-    nbytes = _hip.workspace_bytes(p, chunk) if chunk else 0
+    chunk, nbytes = _split_and_workspace(p, q.dtype, hint, q.device)
     p.q = p.k = p.v = p.o = p.cu_seqlens_q = p.cu_seqlens_k = p.alibi_slopes = None
     return p, chunk, nbytes
+
+
+def _on(device):
+    """Context with `device`, a call's, as the current one: the library plans for
+    the current device's CU count."""
+    if device.type != "cuda" or device.index == torch.cuda.current_device():
+        return contextlib.nullcontext()
+    return torch.cuda.device(device)
+
+
+def _split_and_workspace(p, dtype, hint, device):
+    """(split-KV request, its workspace bytes) of a call on `device`."""
+    with _on(device):
+        chunk = _split_choice(p, dtype, hint)
+        return chunk, _hip.workspace_bytes(p, chunk) if chunk else 0
 
 
 def _split_choice(p, dtype, hint):
@@ -658,7 +672,8 @@ def _prepare_bwd(ts, grads, gdt, batch, Hq, Hkv, Lq, Lk, Dp, varlen, scale, caus
     if alibi_bstride is not None:
         p.alibi_slopes = 256
         p.alibi_batch_stride = alibi_bstride
-    nbytes = _hip.bwd_workspace_bytes(bp)
+    with _on(q.device):
+        nbytes = _hip.bwd_workspace_bytes(bp)
     p.alibi_slopes = p.cu_seqlens_q = p.cu_seqlens_k = None
     return bp, nbytes
 

@@ -16,7 +16,7 @@ import pytest
 import torch
 
 import mtlflashattn_amd as mfa
-from mtlflashattn_amd import _kernel
+from mtlflashattn_amd import _hip, _kernel
 
 
 def t(*shape, dtype=torch.float16):
@@ -377,3 +377,50 @@ class TestLauncherAlignment:
         _kernel._run(q, q, q, out, scale=0.125, causal=False, softcap=0.0, window_left=-1, window_right=-1,
                      alibi=None, alibi_bstride=0)
         assert launches[-1].o % 16 == 0 and launches[-1].o != out.data_ptr()
+
+
+class OnSecondGpu(torch.Tensor):
+    device = property(lambda self: torch.device("cuda", 1))
+
+
+def test_workspaces_are_sized_on_the_tensors_device(monkeypatch):
+    # The size may depend on the device's CU count, and a kept plan is used for
+    # every later call of its signature: whatever device is current when the
+    # plan is made, the library is asked with the tensors' one current.
+    current, asked = [0], []
+
+    class Device:
+        def __init__(self, device):
+            self.index = device.index
+
+        def __enter__(self):
+            current.append(self.index)
+
+        def __exit__(self, *exc):
+            current.pop()
+
+    monkeypatch.setattr(torch.cuda, "device", Device)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[-1])
+    for name, value in (("split_request", 2048), ("workspace_bytes", 4096), ("bwd_workspace_bytes", 4096)):
+        monkeypatch.setattr(_hip, name, lambda *a, name=name, value=value: asked.append((name, current[-1])) or value)
+    launched = []
+    monkeypatch.setattr(_kernel, "_launch", lambda p, chunk, device: launched.append((chunk, p.workspace)))
+    monkeypatch.setattr(_kernel, "_launch_bwd", lambda bp, nbytes, device: launched.append(nbytes))
+    monkeypatch.setattr(_kernel, "_check_device", lambda *a: None)
+    monkeypatch.setattr(_kernel, "_abi_operand", lambda t: tensor())
+    _kernel._plans.clear()
+    _kernel._bwd_plans.clear()
+
+    def tensor(off=0):
+        return torch.zeros(off + 2 * 16 * 4 * 64, dtype=torch.bfloat16)[off:].view(2, 16, 4, 64).as_subclass(OnSecondGpu)
+    kw = dict(scale=0.125, causal=False, softcap=0.0, window_left=-1, window_right=-1, alibi=None, alibi_bstride=0)
+    for off in (0, 1):  # a prepared plan, and an operand that is copied
+        q = tensor(off)
+        _kernel._run(q, q, q, tensor(), **kw)
+    lse = torch.zeros(2, 4, 16).as_subclass(OnSecondGpu)
+    _kernel._run_bwd(*(tensor() for _ in range(5)), lse, into=tuple(tensor() for _ in range(3)), **kw)
+    assert launched == [(2048, 4096), (2048, 4096), 4096]
+    assert {n for n, _ in asked} == {"split_request", "workspace_bytes", "bwd_workspace_bytes"}
+    assert all(device == 1 for _, device in asked), asked
+    _kernel._plans.clear()
+    _kernel._bwd_plans.clear()
