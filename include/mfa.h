@@ -264,9 +264,12 @@ int mfa_fwd_splitkv(const mfa_fwd_params* params, int32_t split_keys, void* work
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  The
  * split-KV partials go to a file-scope device array of
- * MFA_STATIC_SCRATCH_BYTES bytes (one per GPU); a call whose
- * mfa_fwd_workspace_bytes exceeds that returns MFA_ERR_INVALID with a
- * message.  Allocates nothing (no hipMalloc, hipFree or allocating library
+ * MFA_STATIC_SCRATCH_BYTES bytes (one per GPU).  Which calls are taken depends
+ * on the request alone: partials of ceil(seqlen_k / split_keys) * batch *
+ * heads_q * seqlen_q rows of head_dim (padded to 32, 64, 96 or 128) floats, and
+ * a float per row rounded up to 256 bytes, have to fit, else MFA_ERR_INVALID
+ * with a message -- also for single rows, whose own chunks count differently
+ * and which are walked, not refused, where theirs do not fit.  Allocates nothing (no hipMalloc, hipFree or allocating library
  * call); the first call on a GPU looks up the array's device address once.
  * Same kernels, chunks and results as mfa_fwd_splitkv (bit for bit);
  * split_keys 0 behaves as mfa_fwd.  Every call on one GPU shares that GPU's

@@ -3295,8 +3295,11 @@ int mfa_fwd_splitkv_static(const mfa_fwd_params* params, int32_t split_keys, voi
     const int rc = make_plan(params, &plan, chip_geometry_of(static_cast<hipStream_t>(stream)), split_keys);
     if (rc != MFA_OK) return rc;
     if (plan.empty) return MFA_OK;
-    // the size of the request's own chunks decides whether the call is taken;
-    // single rows whose partials are larger than the scratch walk their chunks
+    // The size of the request's own chunks decides whether the call is taken,
+    // also for single rows, which are chunked by their own lengths: the entry
+    // point takes and refuses the same calls whatever the library does with
+    // them.  Single rows whose partials are larger than the scratch walk their
+    // chunks.
     const mfa_fwd_params* p = params;
     const int64_t rows = ((int64_t)p->seqlen_k + split_keys - 1) / split_keys * p->batch * p->heads_q * p->seqlen_q;
     const int dp = padded_dim(p->head_dim);
@@ -3304,9 +3307,9 @@ int mfa_fwd_splitkv_static(const mfa_fwd_params* params, int32_t split_keys, voi
     if (plan.dec_bytes && plan.ws_bytes > MFA_STATIC_SCRATCH_BYTES) walk_single_rows(&plan);
     if (need > MFA_STATIC_SCRATCH_BYTES)
         return set_err(MFA_ERR_INVALID,
-                       "mfa_fwd_splitkv_static: this call needs %lld bytes of workspace, more than the static "
+                       "mfa_fwd_splitkv_static: %lld bytes of partials in chunks of %d keys, more than the static "
                        "scratch's %lld; use mfa_fwd_splitkv with a caller workspace, or larger chunks",
-                       (long long)need, (long long)MFA_STATIC_SCRATCH_BYTES);
+                       (long long)need, split_keys, (long long)MFA_STATIC_SCRATCH_BYTES);
     const hipStream_t st = static_cast<hipStream_t>(stream);
     void* ws = nullptr;
     const int src = static_scratch(st, &ws);

@@ -461,6 +461,18 @@ def test_mixed_calls_have_a_workspace_for_their_single_rows(lib):
     assert b"needed" in lib.mfa_last_error()
 
 
+@pytest.mark.parametrize("lq", [1, 3])
+def test_static_calls_are_refused_by_the_size_of_their_request(lib, lq):
+    # (refused at planning time: nothing is launched)
+    p = good_params(B=64, L=4096, H=64, Hkv=64, D=128)
+    p.seqlen_q, p.seqlen_k = lq, 65536
+    rows = 32 * 64 * 64 * lq
+    need = rows * 128 * 4 + -(-rows * 4 // 256) * 256
+    assert lib.mfa_fwd_splitkv_static(ctypes.byref(p), 2048, None) == _hip.MFA_ERR_INVALID
+    msg = lib.mfa_last_error().decode()
+    assert f"{need} bytes of partials in chunks of 2048 keys" in msg and str(64 << 20) in msg
+
+
 def test_split_kv_workspace_size(lib):
     p = good_params(B=2, L=3000, H=8, Hkv=2, D=64)
     p.seqlen_q = 3
