@@ -150,9 +150,9 @@ __device__ __forceinline__ void store_lse(const KArgs& f, const Unit& u, int r, 
 
 // One K and one V tile of LDS per wavefront: the next K loads run behind the
 // softmax and PV, the next V behind QK.  Two of each, loading two steps ahead,
-// measured slower wherever bandwidth counts (24 sequences to 4096 keys, Hq=32
-// Hkv=8 D=128, two chunks per workgroup: 66.6 against 56.0 us; B=64 Lk=4096 the
-// same: 187.8 and 186.6): with 64 KB at head dim 128 two workgroups share a CU,
+// measured slower wherever bandwidth counts (with plain loads, 24 sequences to
+// 4096 keys, Hq=32 Hkv=8 D=128, two chunks per workgroup: 66.6 against 56.0 us;
+// B=64 Lk=4096 the same: 187.8 and 186.6): with 64 KB at head dim 128 two workgroups share a CU,
 // and one streams while the other starts, merges or ends.
 template <int DP, bool IS_BF16, bool PAGED>
 __global__ void __launch_bounds__(kDecodeThreads) mfa_fwd16x_kernel(DArgs a) {

@@ -2578,23 +2578,33 @@ ChipGeom chip_geometry_current() { return chip_geometry_of(nullptr); }
 // us, a chunk in a walk 2.5), and wins for at most two chunks and in dense calls
 // whose units come out close to whole rounds of one per CU (at head dims up to
 // 64, where a CU takes more of them at once, from two per CU); ragged sequences
-// end too far apart.  Measured (bf16, us per call; chunks per workgroup 1 / 2 / 4 /
-// all; Hq=32 Hkv=8 D=128 where not said):
-//   B=1 Lk=3001 (8 units)                 12.0 / 14.6 / 20.3 / 38.0
-//   B=1 Lk=512 D=64                        7.7 /  6.6 (all)
-//   B=8 Lk=4096 (64 units)                35.7 / 36.5 / 35.2 / 67.9
-//   B=16 (128)                            61.8 / 59.9 / 58.1 / 72.4
-//   B=24 (192)                            89.5 / 87.6 / 86.0 / 82.2
-//   B=32 (256)                           114.5 / 111.6 / 110.3 / 97.6
-//   B=33 (264)                           121.1 / 117.8 / 121.8 / 141.4
-//   B=48 (384)                           173.5 / 165.5 / 163.3 / 159.3
-//   B=1 Lk=128K H=16 (16)                191.1 / 192.1 / 189.8 / 1470
-//   B=48 Lk=6000 Hq=32 Hkv=4 D=64 (192)   65.8 / 67.4 / 70.0 / 78.7
-//   B=64 Lk=4096 H=16 D=64 (1024)        215.1 / 218.3 / 218.2 / 201.2
+// end too far apart (of at most four chunks they would not: below).  Measured
+// with plan_decode's choice of loads (bf16, us of GPU time per call, twenty calls
+// in a graph; chunks per workgroup 1 / 2 / 4 / all; Hq=32 Hkv=8 D=128 where not
+// said):
+//   B=1 Lk=3001 (8 units)                  9.9 / 12.7 / 18.4 / 36.8
+//   B=1 Lk=512 H=16 D=64 (16)              8.1 /  7.0 (all)
+//   B=1 Lk=1024 (8)                        9.6 / 12.3 / 14.7 (all)
+//   B=6 Lk=1500 H=16 D=64 (96)            13.4 / 14.2 / 16.7 / 16.7
+//   B=8 Lk=4096 (64)                      29.3 / 28.8 / 28.8 / 64.1
+//   B=16 (128)                            54.4 / 51.0 / 50.2 / 67.6
+//   B=24 (192)                            77.6 / 75.8 / 74.7 / 72.8
+//   B=32 (256)                           101.4 / 98.8 / 97.0 / 84.3
+//   B=33 (264)                           108.1 / 106.9 / 111.0 / 128.3
+//   B=48 (384)                           153.5 / 149.9 / 148.1 / 140.6
+//   B=64 (512)                           206.5 / 201.3 / 198.6 / 165.7
+//   B=1 Lk=128K (8)                       91.0 / 90.1 / 119.7 / 1458
+//   B=1 Lk=128K H=16 D=64 (16)           100.1 / 100.1 / 91.6 / 1043
+//   B=48 Lk=6000 Hq=32 Hkv=4 D=64 (192)   60.8 / 61.4 / 63.6 / 67.7
+//   B=16 Lk=4096 H=16 D=64 (256)          50.1 / 50.5 / 50.4 / 48.3
+//   B=64 Lk=4096 H=16 D=64 (1024)        192.8 / 193.6 / 197.3 / 187.3
 //   varlen, lengths uniform in [max/16, max]:
-//   24 sequences to 4096 (192)            56.7 / 56.0 / 60.7 / 70.2
-//   64 to 4096 (512)                     138.5 / 134.0 / 136.2 / 140.2
-//   48 to 8192, H=16 D=64 (768)          185.9 / 187.3 / 190.2 / 212.7
+//   24 sequences to 4096 (192)            50.4 / 49.8 / 51.4 / 66.4
+//   64 to 4096 (512)                     118.0 / 113.3 / 113.3 / 127.5
+//   48 to 8192, H=16 D=64 (768)          152.7 / 153.3 / 157.1 / 187.8
+//   16 to 16384 (128)                    150.2 / 143.0 / 143.2 / 246.6
+//   32 to 2048 (256)                      39.7 / 39.8 / 39.5 / 37.3
+//   48 to 1024 (384)                      31.5 / 32.4 / 28.6 / 28.4
 // Calls that mix single rows with longer ones count every sequence as a unit
 // (Hq=32 Hkv=8 D=128, us, all chunks in one workgroup -> this rule): 1 and 4 rows
 // in turn over 32K keys, 2 sequences 477 -> 106, 8 639 -> 341; a 2048-row prefill
