@@ -243,12 +243,15 @@ def _varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, softmax_scale, causal, window_s
         _check_block_table(block_table, lens_k, k.shape[1], k.shape[0])
 
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(q.shape[-1])
+    max_q, max_k = max(lens_q, default=0), max(lens_k, default=0)
     # (with no sequence of exactly one query row, the launch for such rows is
-    # skipped; with none over more than a few keys, no workspace is taken for them)
+    # skipped; beside longer rows and with few keys, no workspace is taken for them)
     single = 1 in lens_q
-    short_single = single and max(b for a, b in zip(lens_q, lens_k) if a == 1) <= _kernel.SHORT_SINGLE_ROW_KEYS
+    few = _kernel.SHORT_SINGLE_ROW_KEYS
+    short_single = (single and max_q > 1 and
+                    (max_k <= few or max(b for a, b in zip(lens_q, lens_k) if a == 1) <= few))
     return forward_varlen(
-        q, k, v, cu_seqlens_q, cu_seqlens_k, max(lens_q, default=0), max(lens_k, default=0),
+        q, k, v, cu_seqlens_q, cu_seqlens_k, max_q, max_k,
         scale=scale, causal=causal, softcap=softcap, window_left=window_size[0],
         window_right=window_size[1], alibi_slopes=alibi_slopes, return_lse=return_lse, block_table=block_table,
         no_single_rows=not single, short_single_rows=short_single, packed=packed,
