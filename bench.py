@@ -372,7 +372,9 @@ def main():
                                    window_right=c["kw"].get("window_size", (-1, -1))[1])
         kname = info.kernel_name.decode()
         chunk = _kernel.split_chunk(c["q"], c["k"])
-        if chunk:
+        if chunk and c["q"].shape[1] == 1:  # (single rows: chunks by their own length)
+            kname += " + mfa_fwd16x_merge"
+        elif chunk:
             kname += f" split-KV {chunk} keys + mfa_combine"
     traffic = None if args.backward else measured_traffic(args.config)
     line = {

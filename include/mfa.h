@@ -53,7 +53,8 @@ extern "C" {
 
 #define MFA_MAX_HEAD_DIM 128
 
-/* tile_hint values (bf16/fp16 only; fp32 has one kernel).  Sequences of one
+/* tile_hint values (bf16/fp16 only; fp32 has two kernels of the same bits, the
+ * library's choice).  Sequences of one
  * query row always run the single-row kernel, which computes the query heads
  * of a K/V head together and whose probabilities carry two 16-bit terms; the
  * hint applies to the rest. */

@@ -2653,11 +2653,11 @@ bool prefer_split32(const mfa_fwd_params* p, int dp, int cus) {
     return whole > (dp <= 64 ? 1.1 : 1.35) * units * (total[1] + 5 * tiles[1]) / (4.0 * cus);
 }
 
-KernelCfg single_cfg(int dp, bool bf16, int lds) {
+KernelCfg single_cfg(int dp, bool bf16) {
     static const char* const names[2][4] = {
         {"mfa_fwd16x<f16,d32>", "mfa_fwd16x<f16,d64>", "mfa_fwd16x<f16,d96>", "mfa_fwd16x<f16,d128>"},
         {"mfa_fwd16x<bf16,d32>", "mfa_fwd16x<bf16,d64>", "mfa_fwd16x<bf16,d96>", "mfa_fwd16x<bf16,d128>"}};
-    return KernelCfg{nullptr, kDecodeRows, 128, lds, names[bf16][dp / 32 - 1], kDecodeThreads};
+    return KernelCfg{nullptr, kDecodeRows, 128, 0, names[bf16][dp / 32 - 1], kDecodeThreads};  // (LDS: plan_decode's)
 }
 
 // The single-row kernel's launch for the call in plan->args: every (sequence,
@@ -2756,9 +2756,9 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
             if (s_in[i] % in_al != 0)
                 return set_err(MFA_ERR_INVALID, "mfa_fwd: q/k/v strides must be multiples of %lld elements",
                                (long long)in_al);
-        // O leaves the 16-bit kernels in row-contiguous 16-byte pieces (and a
-        // packed grouped-query decode uses the head stride as its row stride),
-        // so every o stride is a multiple of 16 bytes, as for q/k/v
+        // O leaves the 16-bit kernels in row-contiguous 16-byte pieces (and
+        // grouped-query tiles pack heads, whose stride is then a row's), so
+        // every o stride is a multiple of 16 bytes, as for q/k/v
         const int64_t out_al = 16 / oes;
         if (p->o_batch_stride % out_al || p->o_seq_stride % out_al || p->o_head_stride % out_al)
             return set_err(MFA_ERR_INVALID, "mfa_fwd: o strides must be multiples of %lld elements (16 bytes)",
@@ -2947,7 +2947,7 @@ int make_plan(const mfa_fwd_params* p, Plan* plan, const ChipGeom& geom, int spl
     if (din == MFA_DTYPE_F32)
         plan->cfg = bias ? select32<true>(dp, split32, paged) : select32<false>(dp, split32, paged);
     else if (single_call)
-        plan->cfg = single_cfg(dp, din == MFA_DTYPE_BF16, 0);  // (its LDS is plan_decode's choice)
+        plan->cfg = single_cfg(dp, din == MFA_DTYPE_BF16);
     else if (tiny_keys && din == MFA_DTYPE_BF16)
         plan->cfg = bias ? select16tk<true, true>(dp) : select16tk<true, false>(dp);
     else if (tiny_keys)

@@ -105,8 +105,12 @@ def _eligibility(q, k, v, attn_mask, dropout_p, is_causal):
         return False, "batch-or-heads-mismatch"
     if k.shape[2] != v.shape[2]:
         return False, "kv-len-mismatch"
-    # fp32 calls that autograd will differentiate stay on stock SDPA (its
-    # gradients flow)
+    # fp32 calls that autograd will differentiate stay on stock SDPA.  The HIP
+    # fp32 backward gives their gradients too, and faster (forward and backward
+    # B=2 H=8 L=1024 D=64 causal 176 us, stock 285; B=1 H=16 L=4096 D=128 causal
+    # 3.0 and 6.1 ms); the gate stays because the patch routes fp32 training
+    # unchanged, bit for bit as without it: who wants it there calls
+    # flash_attn_func.
     if q.dtype == torch.float32 and torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v)):
         return False, "grad-fp32"
     Lq, Lk = q.shape[2], k.shape[2]
