@@ -160,6 +160,14 @@ __device__ __forceinline__ void lds_load16(uint64_t base, uint32_t bytes, uint16
                      : "memory");
 }
 
+// at most N of this wavefront's vector memory operations are still in flight
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// every LDS read of this wavefront has returned: its tile may be overwritten
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 // Compile-time loop: f(std::integral_constant<int, I>{}) for I = 0 .. N-1.
 template <class F, int... I>
 __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {

@@ -34,12 +34,6 @@ namespace {
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 constexpr float kDLn2 = 0.6931471805599453f;
 
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
 // max over the four 16-lane groups (each lane of a group is one query column)
 __device__ __forceinline__ float max_groups(float x) {
     auto a = __builtin_amdgcn_permlane16_swap(__float_as_int(x), __float_as_int(x), false, false);

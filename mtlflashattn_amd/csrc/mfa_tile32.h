@@ -12,13 +12,6 @@
 
 namespace {
 
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-// every LDS read of this wavefront has returned: its tile may be overwritten
-__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
 __device__ __forceinline__ f32x16_t mfma32(float x, float y, const f32x16_t& acc) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc, 0, 0, 0);
 }
