@@ -83,3 +83,17 @@ def test_rows_beyond_32_bit_offsets():
         ts = [q, k, v, dout]
         ts[i] = wide(ts[i])
         assert all(torch.equal(a, b) for a, b in zip(bwd(*ts), ref)), i
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_gradients_do_not_depend_on_the_batch(d):
+    # (the forward's two kernels give the same output and log-sum-exp, and the
+    # backward's order of sums is the sequence's own)
+    q, k, v = make_qkv(40, 256, 256, 8, 2, d, torch.float32, seed=d)
+    dout = torch.randn(q.shape, device=DEV)
+    names = [_kernel.launch_info(t[:n], u[:n], u[:n], causal=True).kernel_name for t, u, n in ((q, k, 40), (q, k, 1))]
+    assert b"split" not in names[0] and b"split" in names[1]
+    whole = grads(q, k, v, dout, causal=True)
+    alone = grads(q[7:8], k[7:8], v[7:8], dout[7:8], causal=True)
+    for a, b in zip(whole, alone):
+        assert torch.equal(a[7:8], b)
