@@ -252,7 +252,8 @@ def _run(q, k, v, out, *, scale, causal, softcap, window_left, window_right, ali
         key = (q.shape, q.stride(), k.shape, k.stride(), v.shape, v.stride(), out.shape, out.stride(), q.dtype,
                out.dtype, q.device.index, float(scale), bool(causal), float(softcap), int(window_left),
                int(window_right), alibi is not None, alibi_bstride,
-               (cu_q.shape[0], Lq, Lk, no_single_rows, short_single_rows) if varlen else None, _TILE_HINT, _SPLIT_KEYS, lse_strides, paged)
+               (cu_q.shape[0], Lq, Lk, no_single_rows, short_single_rows) if varlen else None, _TILE_HINT, _SPLIT_KEYS,
+               lse_strides, paged)
         ent = _plans.get(key)
         if ent is None and all(_fits_strides(t) for t in (q, k, v, out)):
             ent = _prepare(q, k, v, out, batch, Hq, Hkv, Lq, Lk, Dp, varlen, scale, causal, softcap, window_left,

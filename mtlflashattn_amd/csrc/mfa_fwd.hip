@@ -2055,33 +2055,33 @@ mfa_fwd32_kernel(KArgs a) {
         swrite(0);
     }
     for (int n = 0; n < nblk;) {
-      bool last;
-      do {
-        const int j = jbeg + it * BN;
-        const int buf = n & 1;
-        const bool more = n + 1 < nblk;
-        int ncls = cls, nit = it + NC;
-        next_class(ncls, nit);
-        if (more) gload(jbeg + nit * BN);
-        __syncthreads();
+        bool last;
+        do {
+            const int j = jbeg + it * BN;
+            const int buf = n & 1;
+            const bool more = n + 1 < nblk;
+            int ncls = cls, nit = it + NC;
+            next_class(ncls, nit);
+            if (more) gload(jbeg + nit * BN);
+            __syncthreads();
 
-        const bool skip = !wave_live || (j + BN - 1 < w_lo_first) || (j > w_hi_last);
-        if (!skip) {
-            const bool masked = !((j >= w_lo_last) && (j + BN - 1 <= w_hi_first));
-            const float* kbuf = smem + buf * K_ELEMS;
-            const float* vbuf = smem + 2 * K_ELEMS + buf * V_ELEMS;
-            if (masked)
-                block(std::true_type{}, kbuf, vbuf, j);
-            else
-                block(std::false_type{}, kbuf, vbuf, j);
-        }
-        last = ncls != cls || !more;
-        if (more) swrite(buf ^ 1);
-        cls = ncls;
-        it = nit;
-        ++n;
-      } while (!last);
-      end_class();
+            const bool skip = !wave_live || (j + BN - 1 < w_lo_first) || (j > w_hi_last);
+            if (!skip) {
+                const bool masked = !((j >= w_lo_last) && (j + BN - 1 <= w_hi_first));
+                const float* kbuf = smem + buf * K_ELEMS;
+                const float* vbuf = smem + 2 * K_ELEMS + buf * V_ELEMS;
+                if (masked)
+                    block(std::true_type{}, kbuf, vbuf, j);
+                else
+                    block(std::false_type{}, kbuf, vbuf, j);
+            }
+            last = ncls != cls || !more;
+            if (more) swrite(buf ^ 1);
+            cls = ncls;
+            it = nit;
+            ++n;
+        } while (!last);
+        end_class();
     }
 
     // fp32 output (out_f32 is implied for fp32 input)
